@@ -79,7 +79,7 @@ __global__ void batch_reset_kernel(unsigned long long *recs, long long n, unsign
 }
 
 template <int RPT, bool MIXED, int U, bool SINGLE, int SELL>
-__device__ void batch_worker(const BatchArgs &a, int pool, int W, int member, int g0, double *scratch, double *q,
+__device__ __forceinline__ void batch_worker(const BatchArgs &a, int pool, int W, int member, int g0, double *scratch, double *q,
                              double *xs)
 {
     __shared__ int s_idx;
@@ -89,7 +89,6 @@ __device__ void batch_worker(const BatchArgs &a, int pool, int W, int member, in
     gsy.gs.ctl = a.ctl;
     gsy.gs.timeout = a.timeout;
     gsy.gs.G = W;
-    gsy.gs.a2a = W <= kGridA2aMax;
     gsy.gs.acq = SELL ? 0 : 1;  // tile-chunk gathers are plain loads, sliced-ELL gathers agent-scope
     gsy.wg = member;
     gsy.epoch = 0;

@@ -42,7 +42,7 @@ __device__ __forceinline__ int chunk_last(int3 h) { return ((unsigned)h.z >> 27)
 
 // Flagged-record grid barrier state.
 struct GridSync {
-    unsigned long long *recs;   // [2][kMaxRed][G + 1] records of 2 x u64 {lo|epoch, hi|epoch}
+    unsigned long long *recs;   // [2][G + 1][kMaxRed] records of 2 x u64 {lo|epoch, hi|epoch}
     unsigned *ctl;              // ctl[0] abort flag
     long long timeout;          // cycles of s_memtime a wait may last
     int G;
@@ -51,12 +51,9 @@ struct GridSync {
     // another workgroup published is itself an agent-scope load (the sliced-ELL gathers),
     // so the L2 keeps the matrix stream from one iteration to the next
     int acq;
-    // 1: every member polls all member records and combines them itself (one hop, no
-    // broadcast); 0: member 0 gathers and broadcasts (grid_sum)
-    int a2a;
 };
-// Largest group that reduces with every member combining all records (GridSync::a2a).
-constexpr int kGridA2aMax = 64;
+// Largest group that reduces in one hop, every member combining all records (grid_sum).
+constexpr int kGridOneHop = 64;
 
 __device__ __forceinline__ void wait_own_stores() { __builtin_amdgcn_s_waitcnt(0x0F70); /* vmcnt(0) */ }
 
@@ -133,6 +130,15 @@ __device__ __forceinline__ unsigned long long phase_now() { return 0; }
 __device__ __forceinline__ void phase_record(int, unsigned long long) {}
 #endif
 
+// Opaque copy of a value: stops the compiler from hoisting per-row addresses of the
+// vector phases out of the iteration loop (it would pin RPT 64-bit addresses per
+// vector in registers for the whole solve).
+__device__ __forceinline__ int opaque(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // Logical workgroup id: consecutive logical ids on the same XCD (dispatch is
 // round-robin over the 8 XCDs), so each XCD owns a contiguous band of rows and
 // the p gathers of neighbouring rows stay inside one L2.
@@ -183,7 +189,8 @@ __device__ __forceinline__ void store_wt(T *p, T v)
 template <int M>
 __device__ __forceinline__ double xor_move(double v)
 {
-    const int addr = ((threadIdx.x & 63) ^ M) << 2;
+    // (opaque: not hoisted out of the solvers' loops into registers of its own)
+    const int addr = ((opaque((int)threadIdx.x) & 63) ^ M) << 2;
     const int lo = __builtin_amdgcn_ds_bpermute(addr, __double2loint(v));
     const int hi = __builtin_amdgcn_ds_bpermute(addr, __double2hiint(v));
     return __hiloint2double(hi, lo);
@@ -239,8 +246,8 @@ template <int K>
 __device__ __forceinline__ void wave_partials(const double (&v)[K], double *part)
 {
     const double w = wave_join<split_width<K>()>(wave_split<K>(v));
-    const int lane = threadIdx.x & 63;
-    if (lane < K) part[lane * 16 + (threadIdx.x >> 6)] = w;
+    const int tid = opaque((int)threadIdx.x), lane = tid & 63;
+    if (lane < K) part[lane * 16 + (tid >> 6)] = w;
 }
 
 // Called by all 64 lanes of one wave after a barrier: lane 16 k returns the block total of
@@ -248,7 +255,7 @@ __device__ __forceinline__ void wave_partials(const double (&v)[K], double *part
 template <int K>
 __device__ __forceinline__ double block_combine(const double *part, int nwv)
 {
-    const int lane = threadIdx.x & 63, k = lane >> 4, i = lane & 15;
+    const int lane = opaque((int)threadIdx.x) & 63, k = lane >> 4, i = lane & 15;
     double w = (k < K && i < nwv) ? part[k * 16 + i] : 0.0;
     w += dpp_move<0x128>(w);  // row_ror:8
     w += dpp_move<0x124>(w);  // row_ror:4
@@ -332,25 +339,66 @@ __device__ __forceinline__ bool poll_record(const GridSync &gs, const unsigned l
     }
 }
 
-// Grid-wide deterministic all-reduce of K doubles with a barrier (gather to member 0,
-// broadcast back).
+// Sum of value k of members m, m + 16, m + 32, m + 48 below G, in that order, each waited
+// for as in poll_record; every load of a poll is in flight together.
+__device__ __forceinline__ bool poll_members(const GridSync &gs, unsigned epoch, int k, int m, long long t0, double &sum)
+{
+    constexpr int NR = kGridOneHop / 16;
+    const unsigned long long *rec = rec_at(gs, epoch, k, m);
+    unsigned long long lo[NR], hi[NR];
+    for (int n = 1;; n++) {
+#pragma unroll
+        for (int j = 0; j < NR; j++)
+            if (j == 0 || m + 16 * j < gs.G) {
+                const unsigned long long *r = rec + (size_t)j * 16 * kMaxRed * 2;
+                lo[j] = __hip_atomic_load(r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                hi[j] = __hip_atomic_load(r + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } else {
+                lo[j] = hi[j] = (unsigned long long)epoch << 32;  // +0.0, ready
+            }
+        bool ready = true;
+#pragma unroll
+        for (int j = 0; j < NR; j++)
+            ready = ready & ((unsigned)(lo[j] >> 32) == epoch) & ((unsigned)(hi[j] >> 32) == epoch);
+        if (ready) break;
+        if (__builtin_readcyclecounter() - t0 > gs.timeout ||
+            (n % kCtlPollStride == 0 && __hip_atomic_load(gs.ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)) {
+            __hip_atomic_store(gs.ctl, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return false;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
+    sum = 0.0;
+#pragma unroll
+    for (int j = 0; j < NR; j++) sum += __longlong_as_double((long long)((lo[j] & 0xffffffffull) | (hi[j] << 32)));
+    return true;
+}
+
+// Grid-wide deterministic all-reduce of K doubles with a barrier.
 //   v[k]        : this thread's partial; on return the grid total (same bits in every
-//                 workgroup: member 0 sums the member records in a fixed order and every
-//                 member takes its result).
+//                 workgroup: the member records are summed in a fixed order).
 //   visibility  : also make the data every member stored with store_wt before the call
 //                 visible to all members after it: each wave waits for its write-through
 //                 stores before the record is published (no L2 write-back is needed), and
 //                 every member invalidates its L2 (agent acquire) once it has the result.
-// Every member publishes one record per value; member 0 polls all of them, the others
-// poll only the broadcast record with K lanes.  Polling every member record from every
-// workgroup put hundreds of thousands of agent-scope loads on a few cache lines and
-// cost about 10 us per reduction at 256 workgroups; two hops with few pollers cost far
-// less.  Small groups (gs.a2a, at most kGridA2aMax members) skip the broadcast: every
-// member polls all records and combines them in member 0's fixed order, so every member
-// computes the same bits.  A failed wait (watchdog, or the abort flag set by another
-// workgroup) travels in the broadcast tag, so every member leaves at the same sync without
-// a further read of the flag; without the broadcast each member's own polls see the abort
-// flag.  Returns false when the group aborts.
+// Every member publishes one record per value.
+// At most kGridOneHop members: wave 0 of every member polls all records (64 lanes are 16
+// members x 4 values, up to four members a lane with their loads in flight together) and
+// combines them in the wave, one memory hop and no LDS round trip between the partials and
+// the result.  Alone on the chip a reduction takes 1.9 us at 64 members and 1.3 at two
+// (3.0 and 1.6 with all waves of the workgroup polling and a block reduction of what they
+// read; 2D Poisson 64^2: 5.0 -> 4.6 us per iteration).
+// More members: member 0 polls all of them and publishes a broadcast record, which the
+// others poll with K lanes.  Polling every member record from every workgroup put hundreds
+// of thousands of agent-scope loads on a few cache lines and cost about 10 us per reduction
+// at 256 workgroups; two hops with few pollers cost far less.  (Two hops over rows and
+// columns of 16 members, without a root, took 2.7 us instead of 3.1 alone on the chip, but
+// the polling of 256 waves slowed the gathers of the members still in their SpMV: 3D
+// Poisson 77x81x83, tile-mixed, 10.2 -> 10.7 us per iteration.)
+// A failed wait (watchdog, or the abort flag set by another workgroup) travels in the
+// broadcast tag, so every member leaves at the same sync without a further read of the flag;
+// without the broadcast each member's own polls see the abort flag.  Returns false when the
+// group aborts.
 template <int K>
 __device__ __forceinline__ bool grid_sum(const GridSync &gs, double (&v)[K], unsigned &epoch, bool visibility, int wg,
                          double *scratch)
@@ -358,84 +406,83 @@ __device__ __forceinline__ bool grid_sum(const GridSync &gs, double (&v)[K], uns
     __shared__ double s_part[kMaxRed * 16];  // per-wave partials of this member
     __shared__ double s_bc[kMaxRed];         // the group result
     __shared__ int s_fail;
-    const int lane = threadIdx.x & 63, nwv = blockDim.x >> 6;
-    // lane 16 k of wave 0 carries value k through the block combines below
-    const int kl = lane >> 4;
-    const bool klead = threadIdx.x < 64 && (lane & 15) == 0 && kl < K;
     const unsigned long long ph0 = phase_now();
     if (visibility) wait_own_stores();
-    if (threadIdx.x == 0) s_fail = 0;
     wave_partials<K>(v, s_part);
+    if (threadIdx.x == 0) s_fail = 0;
     __syncthreads();
     epoch++;
-    const int G = gs.G;
-    if (G == 1) {
-        // the workgroup is the grid: its barrier is the grid barrier (each wave waited for
-        // its write-through stores before it), and an L1 invalidate makes them visible
-        if (threadIdx.x < 64) {
-            const double m = block_combine<K>(s_part, nwv);
-            if (klead) s_bc[kl] = m;
-        }
-        if (visibility && gs.acq && threadIdx.x < 64) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < K; k++) v[k] = s_bc[k];
-        __syncthreads();
-        return true;
-    }
+    // the lane numbers below are opaque: hoisted out of the solver's iteration loop, the
+    // record addresses would hold registers across the SpMV
+    const int tid = opaque((int)threadIdx.x), nwv = blockDim.x >> 6, G = gs.G;
+    // wave 0 combines the wave partials in a fixed order (lane 16 k: value k) and publishes
+    // this member's record; with visibility every wave has waited for its write-through
+    // stores before the barrier above, so they are complete
+    const int kl = tid >> 4;
+    const bool klead = tid < 64 && (tid & 15) == 0 && kl < K;
     const long long t0 = __builtin_readcyclecounter();
-    // wave 0 combines the wave partials in a fixed order and publishes this member's
-    // record; with visibility every wave has waited for its write-through stores before
-    // the barrier above, so they are complete
-    if (threadIdx.x < 64) {
-        const double m = block_combine<K>(s_part, nwv);
-        if (klead) put_record(rec_at(gs, epoch, kl, wg), m, epoch);
+    if (tid < 64) {
+        double t = block_combine<K>(s_part, nwv);
+        if (G == 1) {
+            // the workgroup is the grid: its barrier is the grid barrier
+            if (klead) s_bc[kl] = t;
+        } else {
+            if (klead) put_record(rec_at(gs, epoch, kl, wg), t, epoch);
+            phase_record(wg, ph0);
+            // keep the compiler from moving the record stores behind this thread's polling
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            if (G <= kGridOneHop) {
+                t = 0.0;
+                bool ok = true;
+                if ((tid & 3) < K && (tid >> 2) < G) ok = poll_members(gs, epoch, tid & 3, tid >> 2, t0, t);
+                t = wave_join<4>(t);
+                if (tid < K) s_bc[tid] = t;
+                if (!ok) s_fail = 1;
+            }
+        }
     }
-    phase_record(wg, ph0);
-    // keep the compiler from moving the record stores behind this thread's polling
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    if (wg == 0 || gs.a2a) {
-        double acc[K];
+    if (G > kGridOneHop) {
+        if (wg == 0) {
+            double acc[K];
 #pragma unroll
-        for (int k = 0; k < K; k++) acc[k] = 0.0;
-        // consecutive threads read a member's K records (adjacent words)
-        for (int i = threadIdx.x; i < K * G; i += blockDim.x) {
-            const int k = i % K;
-            double d;
-            if (!poll_record(gs, rec_at(gs, epoch, k, i / K), epoch, t0, d)) {
-                s_fail = 1;
-                break;
-            }
+            for (int k = 0; k < K; k++) acc[k] = 0.0;
+            // consecutive threads read a member's K records (adjacent words)
+            for (int i = tid; i < K * G; i += blockDim.x) {
+                const int k = i % K;
+                double d;
+                if (!poll_record(gs, rec_at(gs, epoch, k, i / K), epoch, t0, d)) {
+                    s_fail = 1;
+                    break;
+                }
 #pragma unroll
-            for (int kk = 0; kk < K; kk++)
-                if (kk == k) acc[kk] += d;
-        }
-        // fixed order: per thread, then per wave (split reduction), then over the waves
-        wave_partials<K>(acc, scratch);
-        __syncthreads();
-        if (threadIdx.x < 64) {
-            const double t = block_combine<K>(scratch, nwv);
-            if (klead) {
-                if (!gs.a2a) put_record(rec_at(gs, epoch, kl, G), t, s_fail ? (epoch | kAbortTag) : epoch);
-                s_bc[kl] = t;
+                for (int kk = 0; kk < K; kk++)
+                    if (kk == k) acc[kk] += d;
             }
-        }
-        // after the broadcast (off the other members' critical path): drop stale L2 lines
-        if (visibility && gs.acq && threadIdx.x < 64) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    } else {
-        if (threadIdx.x < K) {
+            // fixed order: per thread, then per wave (split reduction), then over the waves
+            wave_partials<K>(acc, scratch);
+            __syncthreads();
+            if (tid < 64) {
+                const double t = block_combine<K>(scratch, nwv);
+                if (klead) {
+                    put_record(rec_at(gs, epoch, kl, G), t, s_fail ? (epoch | kAbortTag) : epoch);
+                    s_bc[kl] = t;
+                }
+            }
+        } else if (tid < K) {
             double d = 0.0;
             bool ab = false;
-            if (!poll_record(gs, rec_at(gs, epoch, threadIdx.x, G), epoch, t0, d, true, &ab) || ab) s_fail = 1;
-            s_bc[threadIdx.x] = d;
+            if (!poll_record(gs, rec_at(gs, epoch, tid, G), epoch, t0, d, true, &ab) || ab) s_fail = 1;
+            s_bc[tid] = d;
         }
-        if (visibility && gs.acq && threadIdx.x < 64) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
+    // (at the root after the broadcast, off the other members' critical path) drop stale
+    // L2 lines
+    if (visibility && gs.acq && threadIdx.x < 64) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < K; k++) v[k] = s_bc[k];
     const bool fail = s_fail != 0;
-    __syncthreads();  // s_part, s_bc and s_fail are rewritten by the next call
+    __syncthreads();  // s_fail is cleared by the next call before its first barrier
     return !fail;
 }
 
@@ -762,15 +809,6 @@ __device__ __forceinline__ int dyn_segment_class(int mode, double p_old, double 
         code = m > 0x1p-13 ? 0 : (m > 0x1p-24 ? 2 : 4);
     }
     return code;
-}
-
-// Opaque copy of a value: stops the compiler from hoisting per-row addresses of the
-// vector phases out of the iteration loop (it would pin RPT 64-bit addresses per
-// vector in registers for the whole solve).
-__device__ __forceinline__ int opaque(int v)
-{
-    asm volatile("" : "+v"(v));
-    return v;
 }
 
 // Rows of this workgroup held by the calling thread: local index t + k*BLK, k < RPT.

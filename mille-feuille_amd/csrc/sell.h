@@ -467,6 +467,13 @@ struct QVec {
         if constexpr (SELL) return reg[k];
         else return lds[loc];
     }
+    // the same for a slot that may lie past the range: 0 there (a sliced-ELL sum of padding
+    // is 0 by itself)
+    __device__ __forceinline__ double row(int k, int loc, bool ok) const
+    {
+        if constexpr (SELL) return reg[k];
+        else return ok ? lds[loc] : 0.0;
+    }
 };
 
 // A row vector of a thread's rows kept in registers (REG) or in the workgroup's LDS slice.
