@@ -213,8 +213,7 @@ typedef struct mf_solve_options {
     int max_replacements;  /* 0 = default 64 */
     int grid;              /* 0 = autotuned; else workgroups (must be co-resident) */
     int block;             /* 0 = default (1024) */
-    int variant;           /* 0 = default (4, or 2 when a workgroup's columns span more than
-                              64 other workgroups or under dynamic classes);
+    int variant;           /* 0 = default (4; 2 under dynamic classes);
                               1 = textbook (3 grid syncs/iteration);
                               2 = fused reductions (2 grid syncs/iteration);
                               3 = pipelined (1 grid sync/iteration);

@@ -78,6 +78,7 @@ struct CgPart {
     int slot;
     NbSync nb;       // publish flags and dependency lists (variant 4)
     int nb_id;       // this workgroup's range: its publish flag and dependency list
+    int wlo, whi;    // kSellWin: the columns [wlo, whi) this workgroup's rows reach
 };
 
 // This workgroup's share of x: in LDS (XREG = false) or in registers (XREG = true).
@@ -102,13 +103,14 @@ struct XVec {
 template <bool MIXED> constexpr int cg_pm() { return MIXED ? kPmLow32 : kPmTiles; }
 
 // q <- A v (tile classes when MIXED) for the vector v published in x64/x32.
-template <bool MIXED, int U, bool DYN, int SELL, int RPT, int BLK>
+// WIN: from the workgroup's LDS window of v.
+template <bool MIXED, int U, bool DYN, int SELL, int RPT, int BLK, int WIN = 0>
 __device__ __forceinline__ void spmv_op(const CgPart &a, Rows<RPT, BLK> &R, const double *x64, const float *x32,
                                         QVec<RPT, (SELL != 0)> &qv, double *scratch)
 {
     if constexpr (SELL != 0) {
-        spmv_sell<MIXED, RPT, BLK, sell_nar(SELL), cg_pm<MIXED>(), sell_vl(SELL, MIXED)>(a.S, a.slot, R.base(), x64,
-                                                                                          x32, qv.reg);
+        spmv_sell<MIXED, RPT, BLK, sell_nar(SELL), cg_pm<MIXED>(), sell_vl(SELL, MIXED), WIN != 0>(
+            a.S, a.slot, R.base() - (WIN ? a.wlo : 0), x64, x32, qv.reg, WIN ? a.S.win_lds : 0);
     } else {
         zero_q<RPT, BLK>(qv.lds, R);
         __syncthreads();
@@ -122,16 +124,57 @@ struct CgResult {
     double rr, bb, rt;
 };
 
-template <int RPT, int BLK>
-__device__ __forceinline__ void publish_p(const CgPart &a, Rows<RPT, BLK> &R, const double (&p)[RPT])
+// Element i of the LDS window of the search direction, binary64 or (W32) its binary32 copy.
+template <bool W32>
+__device__ __forceinline__ void win_put(const CgPart &a, int i, double v)
+{
+    unsigned *w = sell_smem_u32 + (a.S.win_lds >> 2);
+    if constexpr (W32) w[i] = __float_as_uint((float)v);
+    else *reinterpret_cast<double *>(&w[2 * i]) = v;
+}
+
+// Publishes p: its own rows into the workgroup's LDS window (WIN: 0 none, 1 binary64, 2
+// binary32), and to memory for the other workgroups unless there are none (alone).
+template <int RPT, int BLK, int WIN = 0>
+__device__ __forceinline__ void publish_p(const CgPart &a, Rows<RPT, BLK> &R, const double (&p)[RPT],
+                                          bool alone = false)
 {
     R.refresh();
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
         if (!R.ok(k)) continue;
         const int row = R.grow(k);
+        if constexpr (WIN != 0) {
+            win_put<WIN == 2>(a, row - a.wlo, p[k]);
+            if (alone) continue;
+        }
         if (a.need64) store_wt(&a.p64[row], p[k]);
         if (a.need32) store_wt(&a.p32[row], (float)p[k]);
+    }
+}
+
+// The window's columns outside this workgroup's own rows: read from the published p
+// (agent-scope loads; every owner's publish is known to be complete), eight in flight a
+// thread, or zero when no other workgroup exists (no column outside the rows then).
+template <int BLK, bool W32>
+__device__ __forceinline__ void win_halo(const CgPart &a, int row0, int nrows)
+{
+    const i32x4 rs = W32 ? sell_rsrc(a.p32, 4, a.n_sys) : sell_rsrc(a.p64, 8, a.n_sys);
+    const int below = row0 - a.wlo, halo = a.whi - a.wlo - nrows;  // elements before the rows, in all
+    const int t = opaque((int)threadIdx.x);
+    constexpr int U = 8;
+    for (int i0 = t; i0 < halo; i0 += U * BLK) {
+        double v[U];
+        int at[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = min(i0 + u * BLK, halo - 1);
+            at[u] = i < below ? i : i + nrows;
+            if constexpr (W32) v[u] = (double)sell_buf_load_f32(rs, a.wlo + at[u], 0, 0, kSellGatherPolicy);
+            else v[u] = sell_buf_load_f64(rs, a.wlo + at[u], 0, 0, kSellGatherPolicy);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) win_put<W32>(a, at[u], v[u]);
     }
 }
 
@@ -151,7 +194,7 @@ __device__ __forceinline__ void classify_segments(const CgPart &a, Rows<RPT, BLK
 
 // r <- b - A x with the binary64 stream (x published to a.x first); p += (r_new - r_old)
 // when fix_p; returns the r'r sum.  One SpMV and two syncs.
-template <int RPT, int BLK, class Sync, bool XREG, int SELL = 0>
+template <int RPT, int BLK, class Sync, bool XREG, int SELL = 0, int WIN = 0>
 __device__ __forceinline__ bool replace_residual(const CgPart &a, Rows<RPT, BLK> &R, Sync &sy, QVec<RPT, (SELL != 0)> &q, double *scratch,
                                  const XVec<RPT, XREG> &xs, double (&r)[RPT], double (&p)[RPT], double &rr, bool fix_p)
 {
@@ -172,7 +215,7 @@ __device__ __forceinline__ bool replace_residual(const CgPart &a, Rows<RPT, BLK>
         r[k] = rt;
         part[0] += rt * rt;
     }
-    if (fix_p) publish_p<RPT, BLK>(a, R, p);
+    if (fix_p) publish_p<RPT, BLK, WIN>(a, R, p);
     if (!sy.template sum<1>(part, true, scratch)) return false;
     rr = part[0];
     return true;
@@ -468,6 +511,8 @@ __device__ __forceinline__ CgResult cg_core_nb(const CgPart &a, Rows<RPT, BLK> &
     res.rt = -1.0;
     PhaseClock pc;  // per-phase timers (empty unless built with them)
     pc.begin(sy.wg);
+    constexpr int WIN = sell_win(SELL) ? (MIXED ? 2 : 1) : 0;
+    const bool alone = WIN != 0 && sy.gs.G == 1;
     double r[RPT], p[RPT];
     if (a.use_x0) spmv_op<false, U, false, SELL>(a, R, a.x, nullptr, q, scratch);
     double part[2] = {0.0, 0.0};
@@ -484,7 +529,7 @@ __device__ __forceinline__ CgResult cg_core_nb(const CgPart &a, Rows<RPT, BLK> &
         part[0] += r[k] * r[k];
         part[1] += bk * bk;
     }
-    publish_p<RPT, BLK>(a, R, p);
+    publish_p<RPT, BLK, WIN>(a, R, p, alone);
     double rr = 0.0, bb = 0.0, rbase = 0.0;
     bool alive = sy.template sum<2>(part, true, scratch);
     if (alive) {
@@ -517,19 +562,28 @@ __device__ __forceinline__ CgResult cg_core_nb(const CgPart &a, Rows<RPT, BLK> &
         sell_prefetch<sell_lead_stream<MIXED>(), RPT, NAR, PM, LDSV>(a.S.s[sell_lead_stream<MIXED>()], a.slot, lead);
     while (alive && res.status == ST_NOTCONV) {
         pc.start();
-        if (!p_visible && !nb_wait(sy.gs, a.nb, a.nb_id, pub)) {
+        if (!alone && !p_visible && !nb_wait(sy.gs, a.nb, a.nb_id, pub)) {
             res.status = ST_TIMEOUT;
             break;
         }
         pc.mark(0);
         p_visible = false;
+        if constexpr (WIN != 0) {
+            // every wave has left the previous SpMV's gathers (the reduction since), and this
+            // workgroup's own rows went into the window when they were published
+            if (!alone) {
+                win_halo<BLK, WIN == 2>(a, R.row0, R.nrows);
+                __syncthreads();
+            }
+        }
         // q = A p
         if constexpr (LEAD) {
-            spmv_sell_lead<MIXED, RPT, BLK, NAR, PM, LDSV>(a.S, a.slot, R.base(), a.p64, a.p32, q.reg, lead);
+            spmv_sell_lead<MIXED, RPT, BLK, NAR, PM, LDSV, WIN != 0>(a.S, a.slot, R.base() - (WIN ? a.wlo : 0), a.p64,
+                                                                     a.p32, q.reg, lead, WIN ? a.S.win_lds : 0);
             sell_prefetch<sell_lead_stream<MIXED>(), RPT, NAR, PM, LDSV>(a.S.s[sell_lead_stream<MIXED>()], a.slot,
                                                                          lead);
         } else {
-            spmv_op<MIXED, U, false, SELL>(a, R, a.p64, a.p32, q, scratch);
+            spmv_op<MIXED, U, false, SELL, RPT, BLK, WIN>(a, R, a.p64, a.p32, q, scratch);
         }
         pc.mark(1);
         double d[4] = {0.0, 0.0, 0.0, 0.0};
@@ -552,7 +606,7 @@ __device__ __forceinline__ CgResult cg_core_nb(const CgPart &a, Rows<RPT, BLK> &
         if (!a.fixed) {
             bool conv = rr <= a.tol2 * bb;
             if (MIXED && res.repl < a.max_repl && (conv || rr < a.delta2 * rbase)) {
-                if (!replace_residual<RPT, BLK, GridOps, XREG, SELL>(a, R, sy, q, scratch, xs, r, p, rr, true)) {
+                if (!replace_residual<RPT, BLK, GridOps, XREG, SELL, WIN>(a, R, sy, q, scratch, xs, r, p, rr, true)) {
                     res.status = ST_TIMEOUT;
                     break;
                 }
@@ -590,8 +644,9 @@ __device__ __forceinline__ CgResult cg_core_nb(const CgPart &a, Rows<RPT, BLK> &
             r[k] -= alpha * qk;
             p[k] = r[k] + beta * p[k];
         }
-        publish_p<RPT, BLK>(a, R, p);
-        nb_signal(a.nb, a.nb_id, ++pub);
+        publish_p<RPT, BLK, WIN>(a, R, p, alone);
+        if (alone) __syncthreads();
+        else nb_signal(a.nb, a.nb_id, ++pub);
         res.it++;
         pc.mark(4);
         pc.iter();
@@ -863,7 +918,8 @@ __global__ __launch_bounds__(BLK) void cg_kernel(CgArgs a)
     R.row0 = tr0 * kTile;
     R.nrows = min(tr1 * kTile, a.A.n) - R.row0;
     // SELL: 0 tile chunks; 1/2 sliced-ELL, wide/narrow unit profile; 3/4 the same with each
-    // range's rows permuted (sorted by length); + kSellLds: value streams held in LDS
+    // range's rows permuted (sorted by length); + kSellLds*: value streams held in LDS;
+    // + kSellWin: p gathered from an LDS window
     R.perm = sell_perm(SELL) ? a.S.perm + (size_t)wg * RPT * BLK : nullptr;
     R.refresh();
     if constexpr (sell_lds(SELL)) {
@@ -899,6 +955,11 @@ __global__ __launch_bounds__(BLK) void cg_kernel(CgArgs a)
     part.slot = __builtin_amdgcn_readfirstlane(wg * (BLK / 64) + (int)(threadIdx.x >> 6));
     part.nb = a.nb;
     part.nb_id = wg;
+    part.wlo = part.whi = 0;
+    if constexpr (sell_win(SELL)) {
+        part.wlo = __builtin_amdgcn_readfirstlane(a.S.win[2 * wg]);
+        part.whi = __builtin_amdgcn_readfirstlane(a.S.win[2 * wg + 1]);
+    }
     CgResult res;
     if constexpr (VAR == 4)
         res = cg_core_nb<RPT, MIXED, BLK, spmv_unroll<RPT, XREG ? 3 : 2>(), XREG, SELL>(part, R, sy, scratch, q, xs);

@@ -59,6 +59,7 @@ static void free_sell(SellLayout *SL)
         free_dev(SL->val[k]);
         free_dev(SL->lmask[k]);
     }
+    for (int w = 0; w < 2; w++) free_dev(SL->win[w]);
     free_dev(SL->perm);
     delete SL;
 }
@@ -531,10 +532,14 @@ static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &
         val[st].assign((size_t)u * 64 * E * mfk::sell_vbytes_host(st), 0);
     }
     bool range_ok = true;
+    std::vector<int> win[2];  // columns each range reaches: binary64 stream, class streams
+    for (int w = 0; w < 2; w++)
+        if (mask & (w ? 0xFu : 1u << mfk::kSellAll64)) win[w].assign(2 * (size_t)R, 0);
 #pragma omp parallel for schedule(dynamic, 4) reduction(&& : range_ok)
     for (int r = 0; r < R; r++) {
         int r0, nr;
         range_of(r, r0, nr);
+        int lo[2] = {r0, r0}, hi[2] = {r0 + nr - 1, r0 + nr - 1};  // the own rows, as padding reaches them
         std::vector<int> rp;
         std::vector<std::pair<int64_t, int64_t>> ent;
         range_rows(ts, P.h_tr[r], P.h_tr[r + 1], r0, nr, rp, ent);
@@ -584,6 +589,11 @@ static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &
                             const int64_t hi = c0 + (U[st].empty() ? 0 : std::max(U[st].back(), 0));
                             shared[st] = lo >= 0 && hi < n;
                         }
+                        if (shared[st] && soff[st][slot + 1] > soff[st][slot]) {
+                            const int w = st == mfk::kSellAll64 ? 0 : 1, c0 = base[0] + 1024 * k, c1 = base[63] + 1024 * k;
+                            lo[w] = std::min(lo[w], std::min(c0, c1) + (U[st].empty() ? 0 : std::min(U[st].front(), 0)));
+                            hi[w] = std::max(hi[w], std::max(c0, c1) + (U[st].empty() ? 0 : std::max(U[st].back(), 0)));
+                        }
                     }
                 }
                 for (int st = 0; st < mfk::kSellStreams; st++) {
@@ -612,6 +622,9 @@ static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &
                         const double x = L.h_ev[e];
                         for (int st : {c, (int)mfk::kSellAll64}) {
                             if (!(mask >> st & 1)) continue;
+                            const int w = st == mfk::kSellAll64 ? 0 : 1;
+                            lo[w] = std::min(lo[w], col);
+                            hi[w] = std::max(hi[w], col);
                             const int E = mfk::sell_e_host(st, SL.narrow);
                             const int p = shared[st] ? (int)(std::lower_bound(U[st].begin(), U[st].end(),
                                                                               col - own[l]) - U[st].begin())
@@ -634,8 +647,18 @@ static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &
                     }
                 }
             }
+        for (int w = 0; w < 2; w++)
+            if (!win[w].empty()) {
+                win[w][2 * r] = lo[w];
+                win[w][2 * r + 1] = hi[w] + 1;
+            }
     }
     if (!range_ok) return MF_ERR_TOO_LARGE;
+    for (int w = 0; w < 2; w++) {
+        SL.max_win[w] = win[w].empty() ? SL.max_win[w] : 0;
+        for (int r = 0; 2 * (size_t)r < win[w].size(); r++)
+            SL.max_win[w] = std::max(SL.max_win[w], win[w][2 * r + 1] - win[w][2 * r]);
+    }
     // waves whose column words agree in every lane of every unit
     std::vector<int> lm[mfk::kSellStreams];
     for (int st = 0; st < mfk::kSellStreams; st++) {
@@ -657,6 +680,8 @@ static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &
         SL.shared_units[st] = su;
     }
     mf_status st = MF_SUCCESS;
+    for (int w = 0; w < 2 && st == MF_SUCCESS; w++)
+        if (!win[w].empty()) st = upload((void **)&SL.win[w], win[w].data(), sizeof(int) * win[w].size(), s);
     for (int k = 0; k < mfk::kSellStreams && st == MF_SUCCESS; k++) {
         if (!(mask >> k & 1)) continue;
         if ((st = upload((void **)&SL.lmask[k], lm[k].data(), sizeof(int) * lm[k].size(), s)) != MF_SUCCESS) break;

@@ -50,8 +50,11 @@ struct SellStream {
 // the class streams' values (tile-mixed SpMV) are copied into LDS at launch and every
 // SpMV reads them from there; bit 4 (kSellLds64): the same for the binary64 stream.  The
 // choice is compile-time per stream: a runtime choice inside the kernel kept both code
-// paths' registers live and spilled (69 VGPRs).
-constexpr int kSellLdsClass = 8, kSellLds64 = 16;
+// paths' registers live and spilled (69 VGPRs).  Bit 5 (kSellWin): the SpMV of the search
+// direction gathers it from a copy in LDS of the columns the workgroup's rows reach (its
+// window; variant 4, cg_core_nb).
+constexpr int kSellLdsClass = 8, kSellLds64 = 16, kSellWin = 32;
+__host__ __device__ constexpr bool sell_win(int SELL) { return (SELL & kSellWin) != 0; }
 __host__ __device__ constexpr bool sell_nar(int SELL) { return (SELL & 7) == 2 || (SELL & 7) == 4; }
 __host__ __device__ constexpr bool sell_perm(int SELL) { return (SELL & 7) >= 3; }
 __host__ __device__ constexpr bool sell_lds(int SELL) { return (SELL & (kSellLdsClass | kSellLds64)) != 0; }
@@ -70,6 +73,11 @@ struct DevSell {
     // that a slice holds rows of similar length), or null: slot t + 1024 k is local row
     // t + 1024 k
     const int *perm;
+    // per range {first, last + 1} column that the streams of the solve's SpMV reach (class
+    // streams or the binary64 one), and the byte offset in LDS of the workgroup's copy of
+    // the search direction over it (kernels with kSellWin)
+    const int *win;
+    int win_lds;
 };
 
 // Entries per lane per unit (E), value bytes and arithmetic class of each stream.  The
@@ -131,13 +139,15 @@ __device__ __forceinline__ i32x4 sell_rsrc(const void *p, int stride, int n)
     return r;
 }
 
-// x as the gathers see it: binary64 and binary32 copies of n elements.
+// x as the gathers see it: binary64 and binary32 copies of n elements, or the LDS window at
+// byte `win` (element 0 is the window's first column).
 struct SellX {
     i32x4 r64, r32;
+    int win;
 };
 __device__ __forceinline__ SellX sell_x(const double *x64, const float *x32, int n)
 {
-    return SellX{sell_rsrc(x64, 8, n), sell_rsrc(x32, 4, n)};
+    return SellX{sell_rsrc(x64, 8, n), sell_rsrc(x32, 4, n), 0};
 }
 
 template <int NW>
@@ -238,13 +248,17 @@ __device__ __forceinline__ int sell_wg_unit0(const SellStream &st, int slot)
 template <int RPT, bool NAR>
 __device__ __forceinline__ void sell_cache_values(const struct DevSell &D, int wg);
 
-template <int S, bool NAR, int PM>
+template <int S, bool NAR, int PM, bool WIN = false>
 __device__ __forceinline__ void sell_gather(SellUnit<S, NAR, PM> &U, int row, const SellX &X)
 {
 #pragma unroll
     for (int j = 0; j < SellUnit<S, NAR, PM>::E; j++) {
         const int col = row + (int)(short)(U.d.w[j >> 1] >> (16 * (j & 1)));
-        if constexpr (SellUnit<S, NAR, PM>::X32) U.xg[j] = sell_buf_load_f32(X.r32, col, 0, 0, kSellGatherPolicy);
+        if constexpr (WIN && SellUnit<S, NAR, PM>::X32)
+            U.xg[j] = __uint_as_float(sell_smem_u32[(X.win >> 2) + col]);
+        else if constexpr (WIN)
+            U.xg[j] = *reinterpret_cast<const double *>(&sell_smem_u32[(X.win >> 2) + 2 * col]);
+        else if constexpr (SellUnit<S, NAR, PM>::X32) U.xg[j] = sell_buf_load_f32(X.r32, col, 0, 0, kSellGatherPolicy);
         else U.xg[j] = sell_buf_load_f64(X.r64, col, 0, 0, kSellGatherPolicy);
     }
 }
@@ -340,10 +354,10 @@ __device__ __forceinline__ void sell_prefetch(const SellStream &st, int slot, Se
 template <int N>
 using DVec = double __attribute__((ext_vector_type(N)));
 
-template <int S, int RPT, int BLK, bool NAR, int PM = kPmTiles, bool LEAD = false, bool VL = false>
+template <int S, int RPT, int BLK, bool NAR, int PM = kPmTiles, bool LEAD = false, bool VL = false, bool WIN = false>
 __device__ __forceinline__ void sell_stream_impl(const SellStream &st, int slot, int rowb, const double *__restrict__ x64,
                                                  const float *__restrict__ x32, double (&q)[RPT],
-                                                 SellLead<S, NAR, PM> *lead = nullptr)
+                                                 SellLead<S, NAR, PM> *lead = nullptr, int win = 0)
 {
     const int lane = threadIdx.x & 63;
     const int *sb = st.soff + (size_t)slot * RPT;
@@ -352,7 +366,8 @@ __device__ __forceinline__ void sell_stream_impl(const SellStream &st, int slot,
     if (u0 > last) return;
     const int ilane = lane & __builtin_amdgcn_readfirstlane(st.lmask[slot]);
     const int uw0 = VL ? sell_wg_unit0<RPT>(st, slot) : 0;
-    const SellX X = sell_x(x64, x32, st.xmax + 1);
+    SellX X = sell_x(x64, x32, st.xmax + 1);
+    X.win = win;
     // ends of the slices not yet closed, in scalar registers (e[0]: the current one)
     int e[RPT];
 #pragma unroll
@@ -378,7 +393,7 @@ __device__ __forceinline__ void sell_stream_impl(const SellStream &st, int slot,
         sell_load<S, NAR, PM, VL>(st, S0, i, lane, ilane, uw0);
         sell_load<S, NAR, PM, VL>(st, S1, min(i + 1, last), lane, ilane, uw0);
     }
-    sell_gather<S, NAR, PM>(S0, rowb, X);
+    sell_gather<S, NAR, PM, WIN>(S0, rowb, X);
     // unit i's sum into acc; when it ends the slice, acc into q[rot] (the index clamped
     // so that no register outside the vector is ever named).  readfirstlane states that
     // rot is wave-uniform, which the compiler does not prove here: it would keep rot in a
@@ -400,7 +415,7 @@ __device__ __forceinline__ void sell_stream_impl(const SellStream &st, int slot,
     auto step = [&](UT &a, UT &nb1, UT &nb2) {
         sell_load<S, NAR, PM, VL>(st, nb2, min(i + 2, last), lane, ilane, uw0);
         __builtin_amdgcn_sched_barrier(0);
-        sell_gather<S, NAR, PM>(nb1, rowb, X);
+        sell_gather<S, NAR, PM, WIN>(nb1, rowb, X);
         __builtin_amdgcn_sched_barrier(0);
         sum_unit(a);
     };
@@ -416,7 +431,7 @@ __device__ __forceinline__ void sell_stream_impl(const SellStream &st, int slot,
     }
     // one or two units left: unit i is gathered in S0, unit i+1's words are in S1
     if (i < last) {
-        sell_gather<S, NAR, PM>(S1, rowb, X);
+        sell_gather<S, NAR, PM, WIN>(S1, rowb, X);
         __builtin_amdgcn_sched_barrier(0);
         sum_unit(S0);
         sum_unit(S1);
@@ -428,12 +443,12 @@ __device__ __forceinline__ void sell_stream_impl(const SellStream &st, int slot,
 }
 
 // One stream's contribution; VL: values from the workgroup's LDS copy.
-template <int S, int RPT, int BLK, bool NAR, int PM = kPmTiles, bool LEAD = false, bool VL = false>
+template <int S, int RPT, int BLK, bool NAR, int PM = kPmTiles, bool LEAD = false, bool VL = false, bool WIN = false>
 __device__ __forceinline__ void sell_stream(const SellStream &st, int slot, int rowb, const double *__restrict__ x64,
                                             const float *__restrict__ x32, double (&q)[RPT],
-                                            SellLead<S, NAR, PM> *lead = nullptr)
+                                            SellLead<S, NAR, PM> *lead = nullptr, int win = 0)
 {
-    sell_stream_impl<S, RPT, BLK, NAR, PM, LEAD, VL>(st, slot, rowb, x64, x32, q, lead);
+    sell_stream_impl<S, RPT, BLK, NAR, PM, LEAD, VL, WIN>(st, slot, rowb, x64, x32, q, lead, win);
 }
 
 template <int RPT, bool NAR>
@@ -501,37 +516,38 @@ struct RowVec {
 template <bool MIXED> constexpr int sell_lead_stream() { return MIXED ? 3 : kSellAll64; }
 
 // VL: the streams this SpMV reads (class streams when MIXED, else the binary64 one) have LDS
-// copies in the workgroup (sell_vl of the kernel's SELL code)
-template <bool MIXED, int RPT, int BLK, bool NAR = false, int PM = kPmTiles, bool LDSV = false>
+// copies in the workgroup (sell_vl of the kernel's SELL code); WIN: x is read from the LDS
+// window at byte win, and rowb counts from the window's first column
+template <bool MIXED, int RPT, int BLK, bool NAR = false, int PM = kPmTiles, bool LDSV = false, bool WIN = false>
 __device__ __forceinline__ void spmv_sell_lead(const DevSell &D, int slot, int rowb, const double *__restrict__ x64,
                                                const float *__restrict__ x32, double (&q)[RPT],
-                                               SellLead<sell_lead_stream<MIXED>(), NAR, PM> &lead)
+                                               SellLead<sell_lead_stream<MIXED>(), NAR, PM> &lead, int win = 0)
 {
 #pragma unroll
     for (int k = 0; k < RPT; k++) q[k] = 0.0;
     if constexpr (MIXED) {
-        sell_stream<3, RPT, BLK, NAR, PM, true, LDSV>(D.s[3], slot, rowb, x64, x32, q, &lead);
-        sell_stream<0, RPT, BLK, NAR, PM, false, LDSV>(D.s[0], slot, rowb, x64, x32, q);
-        sell_stream<1, RPT, BLK, NAR, PM, false, LDSV>(D.s[1], slot, rowb, x64, x32, q);
-        sell_stream<2, RPT, BLK, NAR, PM, false, LDSV>(D.s[2], slot, rowb, x64, x32, q);
+        sell_stream<3, RPT, BLK, NAR, PM, true, LDSV, WIN>(D.s[3], slot, rowb, x64, x32, q, &lead, win);
+        sell_stream<0, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[0], slot, rowb, x64, x32, q, nullptr, win);
+        sell_stream<1, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[1], slot, rowb, x64, x32, q, nullptr, win);
+        sell_stream<2, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[2], slot, rowb, x64, x32, q, nullptr, win);
     } else {
-        sell_stream<4, RPT, BLK, NAR, PM, true, LDSV>(D.s[4], slot, rowb, x64, x32, q, &lead);
+        sell_stream<4, RPT, BLK, NAR, PM, true, LDSV, WIN>(D.s[4], slot, rowb, x64, x32, q, &lead, win);
     }
 }
 
-template <bool MIXED, int RPT, int BLK, bool NAR = false, int PM = kPmTiles, bool LDSV = false>
+template <bool MIXED, int RPT, int BLK, bool NAR = false, int PM = kPmTiles, bool LDSV = false, bool WIN = false>
 __device__ __forceinline__ void spmv_sell(const DevSell &D, int slot, int rowb, const double *__restrict__ x64,
-                                          const float *__restrict__ x32, double (&q)[RPT])
+                                          const float *__restrict__ x32, double (&q)[RPT], int win = 0)
 {
 #pragma unroll
     for (int k = 0; k < RPT; k++) q[k] = 0.0;
     if constexpr (MIXED) {
-        sell_stream<0, RPT, BLK, NAR, PM, false, LDSV>(D.s[0], slot, rowb, x64, x32, q);
-        sell_stream<1, RPT, BLK, NAR, PM, false, LDSV>(D.s[1], slot, rowb, x64, x32, q);
-        sell_stream<2, RPT, BLK, NAR, PM, false, LDSV>(D.s[2], slot, rowb, x64, x32, q);
-        sell_stream<3, RPT, BLK, NAR, PM, false, LDSV>(D.s[3], slot, rowb, x64, x32, q);
+        sell_stream<0, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[0], slot, rowb, x64, x32, q, nullptr, win);
+        sell_stream<1, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[1], slot, rowb, x64, x32, q, nullptr, win);
+        sell_stream<2, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[2], slot, rowb, x64, x32, q, nullptr, win);
+        sell_stream<3, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[3], slot, rowb, x64, x32, q, nullptr, win);
     } else {
-        sell_stream<4, RPT, BLK, NAR, PM, false, LDSV>(D.s[4], slot, rowb, x64, x32, q);
+        sell_stream<4, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[4], slot, rowb, x64, x32, q, nullptr, win);
     }
 }
 

@@ -22,7 +22,7 @@
 //            w for the iteration's SpMV.
 // variant 4: one grid reduction ({p'q, r'q, q'q, r'r}) per iteration; the publish of p
 //            waits only for the flags of the workgroups owning this one's columns (see
-//            cg_core_nb).  The default when no workgroup depends on more than 64 others.
+//            cg_core_nb).  The default.
 // Mixed precision: the SpMV reads every tile at its storage class with binary32
 // products (p converted to binary32 by its owner when published); x, r, the dot
 // products and scalars stay binary64.  The residual is replaced by b - A x computed
@@ -63,8 +63,12 @@ namespace mf {
 
 using CgKernel = void (*)(mfk::CgArgs);
 
-// Variant 4 by default while no workgroup waits on more than this many others.
-constexpr int kAutoMaxDeps = 64;
+// Systems of at most this many rows and entries run on one workgroup by default, p gathered
+// from LDS: no reduction or publish leaves the CU.  2D Laplacian in binary64, us per
+// iteration on 1 / 64 workgroups: 31 x 33 3.0 / 4.3, 45 x 45 4.3 / 4.6; 3D 12 x 13 x 13
+// tile-mixed 4.7 / 6.0.  Above, one CU's SpMV takes longer than the exchanges it saves (3D
+// 16 x 16 x 16 tile-mixed 5.4 / 5.2, 2D 80 x 80 7.0 / 4.8).
+constexpr int kTinyRows = 2048, kTinyNnz = 16384;
 
 // Rows per thread and block size: 1024 threads, up to 8 rows per thread (r and p in
 // at most 128 VGPRs per wave, 16 waves per CU).
@@ -104,19 +108,25 @@ static CgKernel cg_sell_mixed_for(int rpt, int var)
     return pick_cg<2, true, false, false, SL>(rpt);
 }
 
-// Kernels for rows permuted within each range (SELL 3/4): variants 2 and 4 at 4 and 8 rows
-// per thread, the shapes of the large irregular matrices the permutation is for.
+// Kernels for rows permuted within each range (SELL 3/4): variants 2 and 4.
 template <int VAR, bool MIXED, int SL>
 static CgKernel pick_cg_perm(int rpt)
 {
     switch (rpt) {
+    case 1: return mfk::cg_kernel<1, VAR, MIXED, 1024, false, false, SL>;
+    case 2: return mfk::cg_kernel<2, VAR, MIXED, 1024, false, false, SL>;
     case 4: return mfk::cg_kernel<4, VAR, MIXED, 1024, false, false, SL>;
     case 8: return mfk::cg_kernel<8, VAR, MIXED, 1024, false, false, SL>;
     default: return nullptr;
     }
 }
 
-static bool cg_perm_supported(int rpt, int var) { return (var == 2 || var == 4) && (rpt == 4 || rpt == 8); }
+// Sorting needs slices to sort into: ranges of about two slices only pay for the indirection (graph
+// Laplacian, us per iteration sorted / in order: 78 rows a range 12.9 / 12.4, 234 rows
+// 15.8 / 20.6, 1,172 rows 41 / 53).
+constexpr int kPermMinRows = 128;
+
+static bool cg_perm_supported(int rpt, int var) { return (var == 2 || var == 4) && rpt <= 8; }
 
 // Variant-4 sliced-ELL kernels whose value streams live in LDS (identity row order).
 static CgKernel cg_sell_lds_kernel_for(int rpt, bool mixed, bool narrow)
@@ -124,6 +134,23 @@ static CgKernel cg_sell_lds_kernel_for(int rpt, bool mixed, bool narrow)
     if (mixed) return narrow ? pick_cg<4, true, false, false, 2 | mfk::kSellLdsClass>(rpt)
                              : pick_cg<4, true, false, false, 1 | mfk::kSellLdsClass>(rpt);
     return pick_cg<4, false, false, false, 1 | mfk::kSellLds64>(rpt);
+}
+
+// Variant-4 sliced-ELL kernels that gather p from an LDS window (lds_values: and hold their
+// value streams in LDS too; identity row order).
+static CgKernel cg_sell_win_kernel_for(int rpt, bool mixed, bool narrow, bool perm, bool lds_values)
+{
+    if (!mixed) {
+        if (lds_values) return pick_cg<4, false, false, false, 1 | mfk::kSellLds64 | mfk::kSellWin>(rpt);
+        return perm ? pick_cg<4, false, false, false, 3 | mfk::kSellWin>(rpt)
+                    : pick_cg<4, false, false, false, 1 | mfk::kSellWin>(rpt);
+    }
+    if (perm) return narrow ? pick_cg<4, true, false, false, 4 | mfk::kSellWin>(rpt)
+                            : pick_cg<4, true, false, false, 3 | mfk::kSellWin>(rpt);
+    if (lds_values) return narrow ? pick_cg<4, true, false, false, 2 | mfk::kSellLdsClass | mfk::kSellWin>(rpt)
+                                  : pick_cg<4, true, false, false, 1 | mfk::kSellLdsClass | mfk::kSellWin>(rpt);
+    return narrow ? pick_cg<4, true, false, false, 2 | mfk::kSellWin>(rpt)
+                  : pick_cg<4, true, false, false, 1 | mfk::kSellWin>(rpt);
 }
 
 // LDS bytes of one range's copy of the value streams a solve reads (class streams 0..3 for
@@ -226,19 +253,22 @@ int default_grid(const mf_matrix *A, int maxG, int cg_rows)
 // ext: run on these buffers instead of the matrix's workspace, building nothing (the
 // partition and SpMV streams must exist from an earlier solve) and allocating nothing
 // (no workspace growth, no timing events: info->time_ms is 0).
+// tiny_ok: a system of kTinyRows may run on one workgroup.
 mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve_options *o, mf_solve_info *info,
-                    hipStream_t s, const WsView *ext = nullptr)
+                    hipStream_t s, const WsView *ext = nullptr, bool tiny_ok = true)
 {
     const bool dyn = o->precision == MF_PREC_MIXED && o->dynamic_precision != 0 && A->L.has_copies;
     const bool mixed = o->precision == MF_PREC_MIXED && (A->L.has_lowp || dyn);
     const int tv = A->tuned_variant[mixed ? 1 : 0];
-    // requested variant (0: automatic -- 4 when every workgroup depends on few others,
-    // else 2); dynamic classes run variant 2
+    // requested variant (0: the default, 4); dynamic classes run variant 2
     const int req = dyn ? 2 : (o->variant >= 1 && o->variant <= 4 ? o->variant : (tv >= 1 && tv <= 4 ? tv : 0));
     if (A->L.tilem == 0) return MF_ERR_INVALID;
     // (pipelined CG holds five row vectors: at most 2 rows per thread, so the chunk rule)
-    const int G = choose_grid(A, o, ((long long)(req ? req : 2) << 8) | (mixed ? 1 : 0),
-                              dyn || req == 3 ? 0 : 1024);
+    const long long tuned = ((long long)(req ? req : 2) << 8) | (mixed ? 1 : 0);
+    const bool tiny = tiny_ok && o->grid == 0 && A->tuned_grid.find(tuned) == A->tuned_grid.end() &&
+                      (o->variant == 0 || o->variant == 4) && !dyn && o->layout != 1 && o->value_cache == 0 &&
+                      A->L.n_rows <= kTinyRows && A->L.nnz <= kTinyNnz;
+    const int G = tiny ? 1 : choose_grid(A, o, tuned, dyn || req == 3 ? 0 : 1024);
     if (G > A->L.tilem) return MF_ERR_INVALID;
     const Partition *P = nullptr;
     mf_status st = MF_SUCCESS;
@@ -247,7 +277,11 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     } else if ((st = A->L.partition(G, s, &P)) != MF_SUCCESS) {
         return st;
     }
-    const int var = req ? req : (P->max_deps <= kAutoMaxDeps ? 4 : 2);
+    // point-to-point publishes by default however many workgroups a range's columns span:
+    // waiting for all 256 flags is still cheaper than a second grid reduction (graph
+    // Laplacians whose ranges reach 80 and 130 others, 20,000 and 60,000 rows: 12.3 and 14.3
+    // us per iteration against 12.9 and 15.8 under variant 2)
+    const int var = req ? req : 4;
     int rpt = 0, B = 0;
     if (!shape_for(P->rows_cap, rpt, B)) return MF_ERR_TOO_LARGE;
     // Static classes: sliced-ELL SpMV with q in registers and x in LDS.  Otherwise the
@@ -279,8 +313,8 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     mfk::DevSell dsell;
     memset(&dsell, 0, sizeof(dsell));
     bool narrow = false;
-    if (sell && (st = ensure_sell(A, P, rpt, mixed, s, &dsell, &narrow, cg_perm_supported(rpt, var), !ext)) !=
-                    MF_SUCCESS)
+    if (sell && (st = ensure_sell(A, P, rpt, mixed, s, &dsell, &narrow,
+                                  cg_perm_supported(rpt, var) && A->L.n_rows > kPermMinRows * G, !ext)) != MF_SUCCESS)
         return st;
     // Tile-mixed solve whose class streams would move about as many bytes as the binary64
     // stream (rows spread over classes pad each class stream): binary64 arithmetic on the
@@ -309,10 +343,40 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
             on_chip = true;
         }
     }
+    // p gathered from an LDS window of the columns the workgroup's rows reach, where it fits
+    // next to what the kernel already holds there.  The gathers of rows without common
+    // column offsets touch a 64-byte sector per entry beyond the L2 (agent scope), which
+    // bounds the SpMV; the window is read in whole lines, once, and the gathers go to LDS
+    // (graph Laplacian of 300,007 rows, 21 entries a row within 8,000: 41 -> 26 us per
+    // iteration).  Where the workgroup's entries are few next to its window, loading it costs
+    // more than it saves: 3.5 columns an entry 14.3 -> 13.1 us, 12 an entry 12.3 -> 13.7.
+    // Stencil waves (shared column offsets) gather whole lines as it is.  A grid of one
+    // workgroup always takes the window: p then never leaves the CU.
+    bool window = false;
+    if (sell && k && var == 4) {
+        const SellLayout &SL = *P->sell;
+        int64_t units = 0, shared = 0;
+        for (int s2 = 0; s2 < mfk::kSellStreams; s2++)
+            if (mixed_arith == (s2 != mfk::kSellAll64)) {
+                units += SL.units[s2];
+                shared += SL.shared_units[s2];
+            }
+        const size_t at = (lds + 15) / 16 * 16;
+        const size_t need = at + (size_t)SL.max_win[mixed_arith] * (mixed_arith ? 4 : 8);
+        CgKernel kw = cg_sell_win_kernel_for(rpt, mixed_arith, narrow, dsell.perm != nullptr, on_chip);
+        const bool reuse = 2 * shared < units && (int64_t)SL.max_win[mixed_arith] <= 4 * (A->L.nnz / G);
+        if (kw && (G == 1 || reuse) && need + 4096 <= (size_t)A->max_lds) {
+            k = kw;
+            lds = need;
+            dsell.win = SL.win[mixed_arith];
+            dsell.win_lds = (int)at;
+            window = true;
+        }
+    }
     if (sell && ((!k && dsell.perm) || (fp64_small && var == 4 && !on_chip))) {
         // the partition's streams were built permuted for another variant, or an all-FP64
         // stream chosen for LDS residency did not fit: tile chunks
-        on_chip = false;
+        on_chip = window = false;
         sell = false;
         mixed_arith = mixed;
         lds = (64 + 2 * (size_t)std::max(P->rows_cap, 1)) * sizeof(double);
@@ -321,6 +385,7 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
             lds = lds_x;
         }
     }
+    if (tiny && !window) return cg_launch(A, d_b, d_x, o, info, s, ext, false);
     if (!sell) k = cg_kernel_for(rpt, var, mixed, xreg, dyn);
     if (!k) return var == 3 ? MF_ERR_UNSUPPORTED : MF_ERR_TOO_LARGE;
 
