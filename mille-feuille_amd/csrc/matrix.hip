@@ -82,6 +82,7 @@ void free_partition(Partition &P)
 void DeviceLayout::release()
 {
     free_dev(chunks);
+    free_dev(d_tr_chunk);
     free_dev(eidx);
     free_dev(v64);
     free_dev(v32);
@@ -91,6 +92,7 @@ void DeviceLayout::release()
     for (auto &kv : parts) free_partition(kv.second);
     parts.clear();
     chunks = nullptr;
+    d_tr_chunk = nullptr;
     eidx = nullptr;
     v64 = nullptr;
     v32 = nullptr;
@@ -318,6 +320,18 @@ mf_status DeviceLayout::build_ranges(const std::vector<int> &cuts, hipStream_t s
     return MF_SUCCESS;
 }
 
+mf_status DeviceLayout::ensure_tile_order(hipStream_t s)
+{
+    if (chunks && d_tr_chunk) return MF_SUCCESS;
+    static_assert(sizeof(long long) == sizeof(int64_t), "tile-row chunk offsets");
+    mf_status st = MF_SUCCESS;
+    if (!chunks) st = upload((void **)&chunks, h_chunks.data(), sizeof(int3) * h_chunks.size(), s);
+    if (st == MF_SUCCESS && !d_tr_chunk)
+        st = upload((void **)&d_tr_chunk, tr_chunk.data(), sizeof(int64_t) * tr_chunk.size(), s);
+    if (st == MF_SUCCESS && hipStreamSynchronize(s) != hipSuccess) st = MF_ERR_HIP;
+    return st;
+}
+
 mfk::DevMatrix DeviceLayout::dev(const Partition &P) const
 {
     mfk::DevMatrix d;
@@ -361,30 +375,66 @@ static void range_rows(const TileStruct &ts, int tr0, int tr1, int r0, int nr, s
                 ent[at[bi * kTile + ts.lrow[e] - r0]++] = {e, t};
 }
 
-// Builds the sliced-ELL streams in `mask` (bit s: stream s) for partition P with rpt
-// rows per thread of 1024-thread workgroups.  Thread slot t + 1024 k of range r holds
-// local row perm[t + 1024 k]; slot (range r, wave v, slice k) covers slots
-// 1024 k + 64 v + [0, 64).
-//   * The permutation is fixed at the first build of the partition: the identity, or each
-//     range's rows stably sorted by length (longest first) when that cuts the padded
-//     binary64 stream by 10 % or more (rows of very different lengths in one slice pad to
-//     the longest).  Slots past the range's rows point at its last row.
+// Decides whether the ranges' rows are sorted by length (longest first, stably) for the
+// streams of partition P: when that cuts the padded binary64 stream by 10 % or more.  Fills
+// SL.permuted and, when sorted, SL.h_perm.
+static void choose_order(const mf_matrix *A, const Partition &P, SellLayout &SL, bool allow_perm)
+{
+    SL.ordered = true;
+    SL.permuted = false;
+    if (!allow_perm || A->rowptr.empty()) return;
+    const int R = P.G, LOC = 1024 * SL.rpt, n = A->L.n_rows;
+    const int *rp = A->rowptr.data();
+    std::vector<double> pad_id(R, 0.0), pad_sorted(R, 0.0);
+    std::vector<std::vector<int>> sorted(R);
+#pragma omp parallel for schedule(dynamic, 4)
+    for (int r = 0; r < R; r++) {
+        const int r0 = P.h_tr[r] * kTile, nr = std::max(0, std::min(P.h_tr[r + 1] * kTile, n) - r0);
+        // counting sort by length, longest first
+        int mx = 0;
+        for (int i = 0; i < nr; i++) mx = std::max(mx, rp[r0 + i + 1] - rp[r0 + i]);
+        std::vector<int> at(mx + 2, 0), ord(nr);
+        for (int i = 0; i < nr; i++) at[mx - (rp[r0 + i + 1] - rp[r0 + i]) + 1]++;
+        for (int l = 0; l <= mx; l++) at[l + 1] += at[l];
+        for (int i = 0; i < nr; i++) ord[at[mx - (rp[r0 + i + 1] - rp[r0 + i])]++] = i;
+        for (int s0 = 0; s0 < nr; s0 += 64) {
+            int mi = 0;
+            for (int l = s0; l < std::min(nr, s0 + 64); l++) mi = std::max(mi, rp[r0 + l + 1] - rp[r0 + l]);
+            const int ms = rp[r0 + ord[s0] + 1] - rp[r0 + ord[s0]];
+            pad_id[r] += (mi + 1) / 2 * 2;
+            pad_sorted[r] += (ms + 1) / 2 * 2;
+        }
+        sorted[r] = std::move(ord);
+    }
+    double pi = 0, ps = 0;
+    for (int r = 0; r < R; r++) {
+        pi += pad_id[r];
+        ps += pad_sorted[r];
+    }
+    SL.permuted = ps < 0.9 * pi;
+    if (!SL.permuted) return;
+    SL.h_perm.assign((size_t)R * LOC, 0);
+    for (int r = 0; r < R; r++) {
+        const int r0 = P.h_tr[r] * kTile, nr = std::max(0, std::min(P.h_tr[r + 1] * kTile, n) - r0);
+        int *pr = SL.h_perm.data() + (size_t)r * LOC;
+        for (int i = 0; i < LOC; i++) pr[i] = i < nr ? sorted[r][i] : std::max(0, nr - 1);
+    }
+}
+
+// Builds the sliced-ELL streams in `mask` (bit s: stream s) on the host for partition P,
+// whose rows are sorted by length, with rpt rows per thread of 1024-thread workgroups (ranges
+// in row order: build_sell_gpu).  Thread slot t + 1024 k of range r holds local row
+// perm[t + 1024 k]; slot (range r, wave v, slice k) covers slots 1024 k + 64 v + [0, 64).
+// Slots past the range's rows point at its last row.
 //   * Pass 1 sizes every slot (longest row of the slice in each stream); the unit profile
 //     of the class streams is then chosen (sell.h); an empty slice between two non-empty
 //     ones gets one zero unit.
 //   * Pass 2 writes each row's entries in tile order at its lane, as offsets from the
 //     lane's slot-0 row, and the padding: zero values at offset of the lane's own row (or
 //     of its slot-0 row for slots past the range).
-//   * Shared column words (identity row order): when the union of a slice's relative
-//     columns (col - row) in a stream fits the slice's units, every row -- and every slot
-//     past the range -- is laid out on that union in ascending order, with zero values
-//     where the row has no entry; then all lanes hold the same column words.  The slice
-//     keeps the plain layout when a row's columns in the stream are not strictly
-//     ascending or an aligned column of some lane falls outside [0, n).
 //   * lmask marks the waves whose column words agree in every lane of every unit (0, the
 //     kernels read lane 0's words) or not (63).
-static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &SL, unsigned mask, bool allow_perm,
-                            hipStream_t s)
+static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &SL, unsigned mask, hipStream_t s)
 {
     const TileStruct &ts = A->ts;
     const std::vector<uint8_t> &cls = A->cls;
@@ -395,47 +445,6 @@ static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &
         r0 = P.h_tr[r] * kTile;
         nr = std::max(0, std::min(P.h_tr[r + 1] * kTile, n) - r0);
     };
-    // ---- row permutation (first build of this partition) ----
-    if (SL.h_perm.empty()) {
-        SL.h_perm.assign((size_t)R * LOC, 0);
-        std::vector<double> pad_id(R, 0.0), pad_sorted(R, 0.0);
-        std::vector<std::vector<int>> sorted(R);
-#pragma omp parallel for schedule(dynamic, 4)
-        for (int r = 0; r < R; r++) {
-            int r0, nr;
-            range_of(r, r0, nr);
-            std::vector<int> len(nr, 0);
-            for (int bi = P.h_tr[r]; bi < P.h_tr[r + 1]; bi++)
-                for (int64_t t = ts.tile_ptr[bi]; t < ts.tile_ptr[bi + 1]; t++)
-                    for (int64_t e = ts.tile_off[t]; e < ts.tile_off[t + 1]; e++) len[bi * kTile + ts.lrow[e] - r0]++;
-            std::vector<int> ord(nr);
-            for (int i = 0; i < nr; i++) ord[i] = i;
-            std::stable_sort(ord.begin(), ord.end(), [&](int a, int b) { return len[a] > len[b]; });
-            for (int s0 = 0; s0 < nr; s0 += 64) {
-                int mi = 0, ms = 0;
-                for (int l = s0; l < std::min(nr, s0 + 64); l++) {
-                    mi = std::max(mi, len[l]);
-                    ms = std::max(ms, len[ord[l]]);
-                }
-                pad_id[r] += (mi + 1) / 2 * 2;
-                pad_sorted[r] += (ms + 1) / 2 * 2;
-            }
-            sorted[r] = std::move(ord);
-        }
-        double pi = 0, ps = 0;
-        for (int r = 0; r < R; r++) {
-            pi += pad_id[r];
-            ps += pad_sorted[r];
-        }
-        SL.permuted = allow_perm && ps < 0.9 * pi;
-        for (int r = 0; r < R; r++) {
-            int r0, nr;
-            range_of(r, r0, nr);
-            int *pr = SL.h_perm.data() + (size_t)r * LOC;
-            for (int i = 0; i < LOC; i++)
-                pr[i] = i < nr ? (SL.permuted ? sorted[r][i] : i) : std::max(0, nr - 1);
-        }
-    }
     std::vector<int> Ls[mfk::kSellStreams], nu[mfk::kSellStreams];  // longest row, units per slot
     for (int k = 0; k < mfk::kSellStreams; k++)
         if (mask >> k & 1) {
@@ -554,48 +563,6 @@ static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &
                     base[l] = r0 + pr[64 * v + l];
                     own[l] = l0 + l < nr ? r0 + pr[l0 + l] : base[l];
                 }
-                // union of the relative columns per stream (own - base is 1024 k in every
-                // lane of the identity order, so aligned rows share their column words)
-                std::vector<int> U[mfk::kSellStreams];
-                bool shared[mfk::kSellStreams] = {false, false, false, false, false};
-                if (!SL.permuted) {
-                    bool asc[mfk::kSellStreams] = {true, true, true, true, true};
-                    for (int l = 0; l < 64 && l0 + l < nr; l++) {
-                        const int lr = pr[l0 + l];
-                        int prev[mfk::kSellStreams] = {INT_MIN, INT_MIN, INT_MIN, INT_MIN, INT_MIN};
-                        for (int i = rp[lr]; i < rp[lr + 1]; i++) {
-                            const int64_t e = ent[i].first, t = ent[i].second;
-                            const int rel = ts.tile_col[t] * kTile + ts.lcol[e] - own[l];
-                            for (int st : {(int)cls[t], (int)mfk::kSellAll64}) {
-                                if (!(mask >> st & 1)) continue;
-                                if (rel <= prev[st]) asc[st] = false;
-                                prev[st] = rel;
-                                U[st].push_back(rel);
-                            }
-                        }
-                    }
-                    for (int st = 0; st < mfk::kSellStreams; st++) {
-                        if (!(mask >> st & 1)) continue;
-                        std::sort(U[st].begin(), U[st].end());
-                        U[st].erase(std::unique(U[st].begin(), U[st].end()), U[st].end());
-                        const int64_t cap =
-                            (int64_t)(soff[st][slot + 1] - soff[st][slot]) * mfk::sell_e_host(st, SL.narrow);
-                        shared[st] = asc[st] && (int64_t)U[st].size() <= cap;
-                        // every aligned column (zero entries and padding included) must be a
-                        // column of the matrix in every lane
-                        for (int l = 0; l < 64 && shared[st]; l++) {
-                            const int64_t c0 = (int64_t)base[l] + 1024 * k;
-                            const int64_t lo = c0 + (U[st].empty() ? 0 : std::min(U[st].front(), 0));
-                            const int64_t hi = c0 + (U[st].empty() ? 0 : std::max(U[st].back(), 0));
-                            shared[st] = lo >= 0 && hi < n;
-                        }
-                        if (shared[st] && soff[st][slot + 1] > soff[st][slot]) {
-                            const int w = st == mfk::kSellAll64 ? 0 : 1, c0 = base[0] + 1024 * k, c1 = base[63] + 1024 * k;
-                            lo[w] = std::min(lo[w], std::min(c0, c1) + (U[st].empty() ? 0 : std::min(U[st].front(), 0)));
-                            hi[w] = std::max(hi[w], std::max(c0, c1) + (U[st].empty() ? 0 : std::max(U[st].back(), 0)));
-                        }
-                    }
-                }
                 for (int st = 0; st < mfk::kSellStreams; st++) {
                     if (!(mask >> st & 1)) continue;
                     const int E = mfk::sell_e_host(st, SL.narrow);
@@ -603,9 +570,7 @@ static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &
                         const int16_t pad = (int16_t)(own[l] - base[l]);
                         for (int uu = soff[st][slot]; uu < soff[st][slot + 1]; uu++)
                             for (int j = 0; j < E; j++) {
-                                const size_t pp = (size_t)(uu - soff[st][slot]) * E + j;
-                                idx[st][((size_t)uu * 64 + l) * E + j] =
-                                    shared[st] ? (int16_t)((pp < U[st].size() ? U[st][pp] : 0) + 1024 * k) : pad;
+                                idx[st][((size_t)uu * 64 + l) * E + j] = pad;
                             }
                     }
                 }
@@ -626,9 +591,7 @@ static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &
                             lo[w] = std::min(lo[w], col);
                             hi[w] = std::max(hi[w], col);
                             const int E = mfk::sell_e_host(st, SL.narrow);
-                            const int p = shared[st] ? (int)(std::lower_bound(U[st].begin(), U[st].end(),
-                                                                              col - own[l]) - U[st].begin())
-                                                     : pos[st][l]++;
+                            const int p = pos[st][l]++;
                             const size_t q = ((size_t)(soff[st][slot] + p / E) * 64 + l) * E + p % E;
                             idx[st][q] = (int16_t)off;
                             uint8_t *d = val[st].data() + q * mfk::sell_vbytes_host(st);
@@ -728,7 +691,8 @@ mf_status ensure_sell(mf_matrix *A, const Partition *Pc, int rpt, bool mixed, hi
     if (!SL.soff[mfk::kSellAll64]) mask |= 1u << mfk::kSellAll64;
     if (mixed && !SL.mixed) mask |= 0xFu;
     if (mask) {
-        mf_status st = build_sell(A, P, SL, mask, allow_perm, s);
+        if (!SL.ordered) choose_order(A, P, SL, allow_perm);
+        mf_status st = SL.permuted ? build_sell(A, P, SL, mask, s) : build_sell_gpu(A, P, SL, mask, s);
         if (st != MF_SUCCESS) {
             free_sell(P.sell);
             P.sell = nullptr;

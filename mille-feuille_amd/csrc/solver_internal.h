@@ -24,7 +24,8 @@ struct SellLayout {
     bool mixed = false;             // streams 0..3 built (stream 4 always)
     bool narrow = false;            // unit profile of streams 1..3 (sell.h)
     bool permuted = false;          // rows sorted by length within each range
-    std::vector<int> h_perm;        // host: local row of each thread slot, per range
+    bool ordered = false;           // the row order of this partition has been decided
+    std::vector<int> h_perm;        // host: local row of each thread slot, per range (permuted)
     int *perm = nullptr;            // device copy when permuted
     int64_t units[mfk::kSellStreams] = {0, 0, 0, 0, 0};
     int *soff[mfk::kSellStreams] = {nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -61,7 +62,8 @@ struct DeviceLayout {
     int64_t nnz = 0, tiles = 0, nchunks = 0, npos = 0;
     std::vector<int64_t> tr_chunk;  // host, tilem+1
     std::vector<int3> h_chunks;     // host copy of the headers in tile order
-    int3 *chunks = nullptr;
+    int3 *chunks = nullptr;         // device copies of h_chunks and tr_chunk (ensure_tile_order)
+    long long *d_tr_chunk = nullptr;
     uint8_t *eidx = nullptr;
     double *v64 = nullptr;
     float *v32 = nullptr;
@@ -93,6 +95,8 @@ struct DeviceLayout {
     // tilem, non-decreasing).  The caller owns the result (free_partition).
     mf_status build_ranges(const std::vector<int> &cuts, hipStream_t s, Partition &P) const;
     mfk::DevMatrix dev(const Partition &P) const;
+    // Uploads the chunk headers in tile order and the tile rows' chunk offsets once.
+    mf_status ensure_tile_order(hipStream_t s);
 };
 
 // Whether the persistent CG kernels with rpt rows per thread can use the sliced-ELL
@@ -107,6 +111,9 @@ bool sell_supported(const mf_matrix *A, int rpt);
 // earlier call built do not cover (rpt, mixed).
 mf_status ensure_sell(mf_matrix *A, const Partition *P, int rpt, bool mixed, hipStream_t s, mfk::DevSell *out,
                       bool *narrow, bool allow_perm, bool build = true);
+// The streams of `mask` built on the GPU, for ranges that keep their row order
+// (sell_build.hip).
+mf_status build_sell_gpu(mf_matrix *A, const Partition &P, SellLayout &SL, unsigned mask, hipStream_t s);
 // Padded bytes of one pass over the built class streams (0..3) and over the binary64
 // stream (4) of P's sliced-ELL layout.
 void sell_bytes(const Partition *P, double *class_streams, double *all64);
