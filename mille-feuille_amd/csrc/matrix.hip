@@ -192,6 +192,7 @@ static mf_status build_layout(const TileStruct &ts, const double *val, const std
         }
     }
     L.max_offset = max_off;
+    L.rows_regular = -1;
     L.has_lowp = any_lowp && !v32.empty();
     L.has_copies = !v32.empty();
     mf_status st;
@@ -1010,10 +1011,22 @@ extern "C" mf_status mf_spmv(mf_matrix *A, const double *d_x, double *d_y, int p
         return st != MF_SUCCESS ? st : mf_spmv(T, d_x, d_y, precision, 0, stream);
     }
     const bool mixed = precision == MF_PREC_MIXED && A->L.has_lowp;
+    // (the tile-chunk path's bound: a range's rows on num_cus workgroups fit their LDS)
+    if ((int64_t)A->L.n_rows * 8 > (int64_t)A->max_lds * A->num_cus) return MF_ERR_TOO_LARGE;
+    RowStreams R;
+    mf_status st = row_streams(A, mixed, s, &R);
+    if (st != MF_SUCCESS) return st;
+    if (R.ok) {
+        if (mixed) {
+            if ((st = A->ws.ensure(A->L.n_cols, 1, s)) != MF_SUCCESS) return st;
+            hipLaunchKernelGGL(mfk::to_f32_kernel, dim3(1024), dim3(256), 0, s, d_x, A->ws.p32, A->L.n_cols);
+        }
+        row_spmv(R, A->L.n_rows, d_x, A->ws.p32, d_y, mixed, mfk::kPmTiles, s);
+        return hipGetLastError() == hipSuccess ? MF_SUCCESS : MF_ERR_HIP;
+    }
     int G = spmv_grid(A);
     const Partition *P;
-    mf_status st = A->L.partition(G, s, &P);
-    if (st != MF_SUCCESS) return st;
+    if ((st = A->L.partition(G, s, &P)) != MF_SUCCESS) return st;
     if ((size_t)P->rows_cap * 8 > (size_t)A->max_lds) return MF_ERR_TOO_LARGE;
     if ((st = A->ws.ensure(A->L.n_cols, G, s)) != MF_SUCCESS) return st;
     mfk::DevMatrix dm = A->L.dev(*P);

@@ -248,7 +248,8 @@ __device__ __forceinline__ int sell_wg_unit0(const SellStream &st, int slot)
 template <int RPT, bool NAR>
 __device__ __forceinline__ void sell_cache_values(const struct DevSell &D, int wg);
 
-template <int S, bool NAR, int PM, bool WIN = false>
+// GP: cache policy of the gathers (kernels that only read what earlier launches wrote use 0)
+template <int S, bool NAR, int PM, bool WIN = false, int GP = kSellGatherPolicy>
 __device__ __forceinline__ void sell_gather(SellUnit<S, NAR, PM> &U, int row, const SellX &X)
 {
 #pragma unroll
@@ -258,8 +259,8 @@ __device__ __forceinline__ void sell_gather(SellUnit<S, NAR, PM> &U, int row, co
             U.xg[j] = __uint_as_float(sell_smem_u32[(X.win >> 2) + col]);
         else if constexpr (WIN)
             U.xg[j] = *reinterpret_cast<const double *>(&sell_smem_u32[(X.win >> 2) + 2 * col]);
-        else if constexpr (SellUnit<S, NAR, PM>::X32) U.xg[j] = sell_buf_load_f32(X.r32, col, 0, 0, kSellGatherPolicy);
-        else U.xg[j] = sell_buf_load_f64(X.r64, col, 0, 0, kSellGatherPolicy);
+        else if constexpr (SellUnit<S, NAR, PM>::X32) U.xg[j] = sell_buf_load_f32(X.r32, col, 0, 0, GP);
+        else U.xg[j] = sell_buf_load_f64(X.r64, col, 0, 0, GP);
     }
 }
 
@@ -354,7 +355,8 @@ __device__ __forceinline__ void sell_prefetch(const SellStream &st, int slot, Se
 template <int N>
 using DVec = double __attribute__((ext_vector_type(N)));
 
-template <int S, int RPT, int BLK, bool NAR, int PM = kPmTiles, bool LEAD = false, bool VL = false, bool WIN = false>
+template <int S, int RPT, int BLK, bool NAR, int PM = kPmTiles, bool LEAD = false, bool VL = false, bool WIN = false,
+          int GP = kSellGatherPolicy>
 __device__ __forceinline__ void sell_stream_impl(const SellStream &st, int slot, int rowb, const double *__restrict__ x64,
                                                  const float *__restrict__ x32, double (&q)[RPT],
                                                  SellLead<S, NAR, PM> *lead = nullptr, int win = 0)
@@ -393,7 +395,7 @@ __device__ __forceinline__ void sell_stream_impl(const SellStream &st, int slot,
         sell_load<S, NAR, PM, VL>(st, S0, i, lane, ilane, uw0);
         sell_load<S, NAR, PM, VL>(st, S1, min(i + 1, last), lane, ilane, uw0);
     }
-    sell_gather<S, NAR, PM, WIN>(S0, rowb, X);
+    sell_gather<S, NAR, PM, WIN, GP>(S0, rowb, X);
     // unit i's sum into acc; when it ends the slice, acc into q[rot] (the index clamped
     // so that no register outside the vector is ever named).  readfirstlane states that
     // rot is wave-uniform, which the compiler does not prove here: it would keep rot in a
@@ -415,7 +417,7 @@ __device__ __forceinline__ void sell_stream_impl(const SellStream &st, int slot,
     auto step = [&](UT &a, UT &nb1, UT &nb2) {
         sell_load<S, NAR, PM, VL>(st, nb2, min(i + 2, last), lane, ilane, uw0);
         __builtin_amdgcn_sched_barrier(0);
-        sell_gather<S, NAR, PM, WIN>(nb1, rowb, X);
+        sell_gather<S, NAR, PM, WIN, GP>(nb1, rowb, X);
         __builtin_amdgcn_sched_barrier(0);
         sum_unit(a);
     };
@@ -431,7 +433,7 @@ __device__ __forceinline__ void sell_stream_impl(const SellStream &st, int slot,
     }
     // one or two units left: unit i is gathered in S0, unit i+1's words are in S1
     if (i < last) {
-        sell_gather<S, NAR, PM, WIN>(S1, rowb, X);
+        sell_gather<S, NAR, PM, WIN, GP>(S1, rowb, X);
         __builtin_amdgcn_sched_barrier(0);
         sum_unit(S0);
         sum_unit(S1);
@@ -443,12 +445,13 @@ __device__ __forceinline__ void sell_stream_impl(const SellStream &st, int slot,
 }
 
 // One stream's contribution; VL: values from the workgroup's LDS copy.
-template <int S, int RPT, int BLK, bool NAR, int PM = kPmTiles, bool LEAD = false, bool VL = false, bool WIN = false>
+template <int S, int RPT, int BLK, bool NAR, int PM = kPmTiles, bool LEAD = false, bool VL = false, bool WIN = false,
+          int GP = kSellGatherPolicy>
 __device__ __forceinline__ void sell_stream(const SellStream &st, int slot, int rowb, const double *__restrict__ x64,
                                             const float *__restrict__ x32, double (&q)[RPT],
                                             SellLead<S, NAR, PM> *lead = nullptr, int win = 0)
 {
-    sell_stream_impl<S, RPT, BLK, NAR, PM, LEAD, VL, WIN>(st, slot, rowb, x64, x32, q, lead, win);
+    sell_stream_impl<S, RPT, BLK, NAR, PM, LEAD, VL, WIN, GP>(st, slot, rowb, x64, x32, q, lead, win);
 }
 
 template <int RPT, bool NAR>
@@ -535,19 +538,20 @@ __device__ __forceinline__ void spmv_sell_lead(const DevSell &D, int slot, int r
     }
 }
 
-template <bool MIXED, int RPT, int BLK, bool NAR = false, int PM = kPmTiles, bool LDSV = false, bool WIN = false>
+template <bool MIXED, int RPT, int BLK, bool NAR = false, int PM = kPmTiles, bool LDSV = false, bool WIN = false,
+          int GP = kSellGatherPolicy>
 __device__ __forceinline__ void spmv_sell(const DevSell &D, int slot, int rowb, const double *__restrict__ x64,
                                           const float *__restrict__ x32, double (&q)[RPT], int win = 0)
 {
 #pragma unroll
     for (int k = 0; k < RPT; k++) q[k] = 0.0;
     if constexpr (MIXED) {
-        sell_stream<0, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[0], slot, rowb, x64, x32, q, nullptr, win);
-        sell_stream<1, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[1], slot, rowb, x64, x32, q, nullptr, win);
-        sell_stream<2, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[2], slot, rowb, x64, x32, q, nullptr, win);
-        sell_stream<3, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[3], slot, rowb, x64, x32, q, nullptr, win);
+        sell_stream<0, RPT, BLK, NAR, PM, false, LDSV, WIN, GP>(D.s[0], slot, rowb, x64, x32, q, nullptr, win);
+        sell_stream<1, RPT, BLK, NAR, PM, false, LDSV, WIN, GP>(D.s[1], slot, rowb, x64, x32, q, nullptr, win);
+        sell_stream<2, RPT, BLK, NAR, PM, false, LDSV, WIN, GP>(D.s[2], slot, rowb, x64, x32, q, nullptr, win);
+        sell_stream<3, RPT, BLK, NAR, PM, false, LDSV, WIN, GP>(D.s[3], slot, rowb, x64, x32, q, nullptr, win);
     } else {
-        sell_stream<4, RPT, BLK, NAR, PM, false, LDSV, WIN>(D.s[4], slot, rowb, x64, x32, q, nullptr, win);
+        sell_stream<4, RPT, BLK, NAR, PM, false, LDSV, WIN, GP>(D.s[4], slot, rowb, x64, x32, q, nullptr, win);
     }
 }
 

@@ -255,10 +255,19 @@ mf_status build_sell_gpu(mf_matrix *A, const Partition &P, SellLayout &SL, unsig
     std::vector<mfk::SellSlot> info((size_t)mfk::kSellStreams * slots);
     DevBuf dinfo;
     if (hipMalloc(&dinfo.p, sizeof(mfk::SellSlot) * info.size()) != hipSuccess) return MF_ERR_ALLOC;
-    hipLaunchKernelGGL(mfk::sell_count_kernel, dim3((unsigned)slots), dim3(64), 0, s, a, mask, (mfk::SellSlot *)dinfo.p);
+    // streams of classes that no tile has stay empty
+    const mfk::SellSlot none{0, 0, 0, 0, INT_MAX, INT_MIN};
+    unsigned counted = mask;
+    for (int k = 0; k < mfk::kSellAll64; k++)
+        if ((mask >> k & 1) && L.nnz_by_class[k] == 0) {
+            counted &= ~(1u << k);
+            std::fill_n(info.begin() + k * slots, slots, none);
+        }
+    hipLaunchKernelGGL(mfk::sell_count_kernel, dim3((unsigned)slots), dim3(64), 0, s, a, counted,
+                       (mfk::SellSlot *)dinfo.p);
     if (hipGetLastError() != hipSuccess) return MF_ERR_HIP;
     for (int k = 0; k < mfk::kSellStreams; k++)
-        if ((mask >> k & 1) &&
+        if ((counted >> k & 1) &&
             hipMemcpyAsync(info.data() + k * slots, (mfk::SellSlot *)dinfo.p + k * slots, sizeof(mfk::SellSlot) * slots,
                            hipMemcpyDeviceToHost, s) != hipSuccess)
             return MF_ERR_HIP;

@@ -72,6 +72,7 @@ struct DeviceLayout {
     int *src = nullptr;             // per entry: position in the input CSR arrays
     std::vector<double> h_ev;       // host: entry values in tile order (sliced-ELL build)
     int max_offset = 0;             // max |col - row| over the entries
+    int rows_regular = -1;          // whether row streams suit the matrix (row_streams; -1: not looked at)
     bool has_lowp = false;
     bool has_copies = false;        // v32/v16/v8 hold every entry (lossy where the class is higher)
     int64_t tiles_by_class[4] = {0, 0, 0, 0};
@@ -118,6 +119,22 @@ mf_status build_sell_gpu(mf_matrix *A, const Partition &P, SellLayout &SL, unsig
 // stream (4) of P's sliced-ELL layout.
 void sell_bytes(const Partition *P, double *class_streams, double *all64);
 
+
+// Sliced-ELL streams over ranges of 1024 rpt consecutive rows for products launched by
+// themselves (sell_spmv.hip), built on first use; ok = false: the matrix keeps the tile chunks
+// (not square, columns beyond the 16-bit offsets, or rows of very different lengths).
+struct RowStreams {
+    bool ok = false;
+    const DeviceLayout *L = nullptr;
+    const Partition *P = nullptr;
+    mfk::DevSell S;
+    bool narrow = false;
+    int rpt = 0;
+};
+mf_status row_streams(mf_matrix *A, bool mixed, hipStream_t s, RowStreams *out);
+// y = A x: binary64 values and x64, or (mixed) the tile classes under product mode pm.
+void row_spmv(const RowStreams &R, int n, const double *x64, const float *x32, double *y, bool mixed, int pm,
+              hipStream_t s);
 
 // Per-matrix solver scratch (vectors, barrier records, status words).
 struct Workspace {

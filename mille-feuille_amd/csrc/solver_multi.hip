@@ -1,8 +1,17 @@
-// Multi-kernel fallback: the same CG / BiCGSTAB recurrences driven by a host loop,
-// one launch per SpMV or BLAS-1 step and one scalar copy to the host per iteration
-// (the structure of cg_solve_reduce, main-cg.cu:258-292, and of the multi-kernel
-// bicgstab, main-bicg.cu:1619-1656).  No co-residency requirement, so it runs any
-// size.  Scalars live on the device; dot products are deterministic two-pass sums.
+// Multi-kernel fallback: CG / BiCGSTAB driven by a host loop (the reference's
+// cg_solve_reduce, main-cg.cu:258-292, and multi-kernel bicgstab, main-bicg.cu:1619-1656).
+// No co-residency requirement, so it runs any size.  Scalars live on the device; dot
+// products are deterministic two-pass sums.
+//
+// CG is two launches an iteration, the recurrence of the persistent kernels' variant 4:
+//   mk_cg_spmv    q = A p and each workgroup's part of {p'q, r'q, q'q, r'r}
+//   mk_cg_update  every workgroup sums the parts, decides alike (convergence, replacement,
+//                 breakdown), and updates x, r and p in one pass
+// The host enqueues kBatch iterations at a time and reads the state once per batch; after a
+// decision the remaining launches of a batch do nothing.  An iteration reads the matrix, 24
+// bytes a row in the product and 32 in the update, and writes 8 and 24 (28 tile-mixed); it
+// took 11 launches, 155 bytes a row and two host synchronisations before (3D 144 x 145 x 147
+// tile-mixed: 204 us, of which the SpMV on tile chunks 80).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -62,6 +71,127 @@ __global__ __launch_bounds__(256) void mk_finish(const double *__restrict__ part
     if (threadIdx.x == 0) *out = s[0] + s[1] + s[2] + s[3];
 }
 
+// State of a multi-kernel CG, in the solve's 32 scalars.
+enum { MKS_RR = 0, MKS_IT = 1, MKS_STATE = 2 };
+enum { MK_RUN = 0, MK_CHECK = 1, MK_BREAK = 2, MK_MAXIT = 3 };
+constexpr int kUpdBlocks = 512, kUpdThreads = 512;
+
+// q = A p over row streams, range blockIdx.x, + gridDim.x, ...; part[4 b ..] = this
+// workgroup's {p'q, r'q, q'q, r'r}.
+template <int RPT, bool MIXED, bool NAR>
+__global__ __launch_bounds__(1024) void mk_cg_spmv(DevSell S, const int *wg_tr, int ranges, int n,
+                                                   const double *__restrict__ p, const float *__restrict__ p32,
+                                                   const double *__restrict__ r, double *__restrict__ q,
+                                                   double *__restrict__ part, const double *sc)
+{
+    __shared__ double scratch[64];
+    if (sc[MKS_STATE] != (double)MK_RUN) return;
+    double d[4] = {0.0, 0.0, 0.0, 0.0};
+    const int b = logical_wg(blockIdx.x, gridDim.x);
+    // a workgroup's ranges are neighbours
+    const int r_lo = (int)((long long)ranges * b / gridDim.x), r_hi = (int)((long long)ranges * (b + 1) / gridDim.x);
+    for (int g = r_lo; g < r_hi; g++) {
+        const int slot = __builtin_amdgcn_readfirstlane(g * 16 + (int)(threadIdx.x >> 6));
+        const int row0 = wg_tr[g] * kTile, nrows = min(wg_tr[g + 1] * kTile, n) - row0;
+        const int t = threadIdx.x;
+        double qv[RPT];
+        spmv_sell<MIXED, RPT, 1024, NAR, MIXED ? kPmLow32 : kPmTiles, false, false, 0>(
+            S, slot, row0 + min(t, nrows - 1), p, p32, qv);
+#pragma unroll
+        for (int k = 0; k < RPT; k++) {
+            const int row = row0 + t + 1024 * k;
+            if (t + 1024 * k >= nrows) continue;
+            const double pk = p[row], rk = r[row], qk = qv[k];
+            q[row] = qk;
+            d[0] += pk * qk;
+            d[1] += rk * qk;
+            d[2] += qk * qk;
+            d[3] += rk * rk;
+        }
+    }
+    block_sum<4>(d, scratch);
+    if (threadIdx.x < 4) part[4 * (size_t)b + threadIdx.x] = threadIdx.x == 0 ? d[0] : threadIdx.x == 1 ? d[1]
+                                                                             : threadIdx.x == 2 ? d[2] : d[3];
+}
+
+// The same sums for a product made by the tile-chunk SpMV.
+__global__ __launch_bounds__(1024) void mk_cg_dots(int n, const double *__restrict__ p, const double *__restrict__ r,
+                                                   const double *__restrict__ q, double *__restrict__ part,
+                                                   const double *sc)
+{
+    __shared__ double scratch[64];
+    if (sc[MKS_STATE] != (double)MK_RUN) return;
+    double d[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const double pk = p[i], rk = r[i], qk = q[i];
+        d[0] += pk * qk;
+        d[1] += rk * qk;
+        d[2] += qk * qk;
+        d[3] += rk * rk;
+    }
+    block_sum<4>(d, scratch);
+    if (threadIdx.x < 4) part[4 * (size_t)blockIdx.x + threadIdx.x] = threadIdx.x == 0 ? d[0] : threadIdx.x == 1 ? d[1]
+                                                                                      : threadIdx.x == 2 ? d[2] : d[3];
+}
+
+// Iteration `it`: the tests of the recurrence on the exact r'r, then x += alpha p,
+// r -= alpha q, p = r + beta p.  check2: r'r at or below which the host has to look (it
+// converged, or a tile-mixed residual is due for replacement); negative: never.  Block 0
+// records the state, which the launches after this one read.
+__global__ __launch_bounds__(kUpdThreads) void mk_cg_update(int n, int nparts, const double *__restrict__ part, double check2,
+                                                            int it, int maxit, double *__restrict__ x,
+                                                            double *__restrict__ r, double *__restrict__ p,
+                                                            float *__restrict__ p32, const double *__restrict__ q,
+                                                            double *sc)
+{
+    __shared__ double scratch[64];
+    if (sc[MKS_STATE] != (double)MK_RUN) return;
+    double d[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int i = threadIdx.x; i < nparts; i += kUpdThreads) {
+        const double2 a = reinterpret_cast<const double2 *>(part)[2 * i], b = reinterpret_cast<const double2 *>(part)[2 * i + 1];
+        d[0] += a.x;
+        d[1] += a.y;
+        d[2] += b.x;
+        d[3] += b.y;
+    }
+    block_sum<4>(d, scratch);
+    const double rr = d[3];
+    const int state = rr <= check2 ? MK_CHECK : it >= maxit ? MK_MAXIT : (!(d[0] != 0.0) || !isfinite(d[0])) ? MK_BREAK : MK_RUN;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc[MKS_RR] = rr;
+        sc[MKS_IT] = (double)it;
+        if (state != MK_RUN) sc[MKS_STATE] = (double)state;
+    }
+    if (state != MK_RUN) return;
+    const double alpha = rr / d[0];
+    double rr_new = rr - 2.0 * alpha * d[1] + alpha * alpha * d[2];
+    if (!(rr_new > 0.0)) rr_new = 0.0;
+    const double beta = rr_new / rr;
+    const int step = 2 * gridDim.x * kUpdThreads;
+    for (int i = 2 * (blockIdx.x * kUpdThreads + threadIdx.x); i + 1 < n; i += step) {
+        double2 xv = *reinterpret_cast<double2 *>(x + i), rv = *reinterpret_cast<double2 *>(r + i);
+        double2 pv = *reinterpret_cast<double2 *>(p + i);
+        const double2 qv = *reinterpret_cast<const double2 *>(q + i);
+        xv.x += alpha * pv.x;
+        xv.y += alpha * pv.y;
+        rv.x -= alpha * qv.x;
+        rv.y -= alpha * qv.y;
+        pv.x = rv.x + beta * pv.x;
+        pv.y = rv.y + beta * pv.y;
+        *reinterpret_cast<double2 *>(x + i) = xv;
+        *reinterpret_cast<double2 *>(r + i) = rv;
+        *reinterpret_cast<double2 *>(p + i) = pv;
+        if (p32) *reinterpret_cast<float2 *>(p32 + i) = make_float2((float)pv.x, (float)pv.y);
+    }
+    if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+        const int i = n - 1;
+        x[i] += alpha * p[i];
+        r[i] -= alpha * q[i];
+        p[i] = r[i] + beta * p[i];
+        if (p32) p32[i] = (float)p[i];
+    }
+}
+
 // Whether every scalar slot named in `mask` (bit k: sc[k]) is finite and nonzero.  The
 // vector updates of an iteration do nothing when a denominator broke down, so the
 // iterate the host finds on MF_BREAKDOWN is the last finite one.
@@ -73,29 +203,6 @@ __device__ __forceinline__ bool mk_ok(const double *sc, unsigned mask)
             if (!(d != 0.0) || !isfinite(d)) return false;
         }
     return true;
-}
-
-// y = a*x + y with a = sc[num]/sc[den] (sign applied); nothing when sc[den] broke down
-__global__ __launch_bounds__(256) void mk_axpy(const double *__restrict__ sc, int num, int den, double sign,
-                                               const double *__restrict__ x, double *__restrict__ y, int n)
-{
-    if (!mk_ok(sc, 1u << den)) return;
-    const double a = sign * sc[num] / sc[den];
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) y[i] += a * x[i];
-}
-
-// p = r + (sc[num]/sc[den]) p, plus binary32 copy; nothing when a slot of `guard` broke down
-__global__ __launch_bounds__(256) void mk_xpay(const double *__restrict__ sc, int num, int den, unsigned guard,
-                                               const double *__restrict__ r, double *__restrict__ p,
-                                               float *__restrict__ p32, int n)
-{
-    if (!mk_ok(sc, guard)) return;
-    const double beta = sc[num] / sc[den];
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const double v = r[i] + beta * p[i];
-        p[i] = v;
-        if (p32) p32[i] = (float)v;
-    }
 }
 
 __global__ void mk_copy(const double *__restrict__ a, double *__restrict__ b, float *__restrict__ b32, int n)
@@ -178,6 +285,7 @@ struct MkCtx {
     int n;
     double *partial = nullptr;
     double *sc = nullptr;
+    RowStreams rows;   // the products' streams, when the matrix suits them (else tile chunks)
     std::vector<void *> bufs;
 
     ~MkCtx()
@@ -195,7 +303,9 @@ struct MkCtx {
     // use_mixed: tile classes with product mode pm (kPmLow32 CG, kPmWide64 BiCGSTAB)
     void spmv(const double *x64, const float *x32, double *y, bool use_mixed, int pm = mfk::kPmLow32)
     {
-        if (use_mixed && pm == mfk::kPmWide64)
+        if (rows.ok)
+            row_spmv(rows, n, x64, x32, y, use_mixed, pm, s);
+        else if (use_mixed && pm == mfk::kPmWide64)
             hipLaunchKernelGGL((mfk::mk_spmv<true, mfk::kPmWide64>), dim3(G), dim3(1024), lds, s, dm, x64, x32, y);
         else if (use_mixed)
             hipLaunchKernelGGL((mfk::mk_spmv<true, mfk::kPmLow32>), dim3(G), dim3(1024), lds, s, dm, x64, x32, y);
@@ -224,6 +334,15 @@ mf_status mk_setup(mf_matrix *A, const mf_solve_options *o, hipStream_t s, MkCtx
     c.n = A->L.n_rows;
     c.mixed = o->precision == MF_PREC_MIXED && A->L.has_lowp;
     if (A->L.tilem == 0 || A->L.n_rows != A->L.n_cols) return MF_ERR_INVALID;
+    mf_status rst = row_streams(A, c.mixed, s, &c.rows);
+    if (rst != MF_SUCCESS) return rst;
+    c.partial = c.alloc<double>(mfk::kDotBlocks);
+    c.sc = c.alloc<double>(32);
+    if (!c.partial || !c.sc) return MF_ERR_ALLOC;
+    if (c.rows.ok) {
+        c.G = c.rows.P->G;
+        return MF_SUCCESS;
+    }
     // at most 4096 rows (32 KB of LDS) per workgroup; any number of workgroups
     int G = std::max(1, std::min(A->L.tilem, std::max(A->num_cus, (A->L.n_rows + 4095) / 4096)));
     mf_status st;
@@ -239,9 +358,6 @@ mf_status mk_setup(mf_matrix *A, const mf_solve_options *o, hipStream_t s, MkCtx
     for (auto k : {(const void *)mfk::mk_spmv<true, mfk::kPmLow32>, (const void *)mfk::mk_spmv<true, mfk::kPmWide64>,
                    (const void *)mfk::mk_spmv<false, mfk::kPmTiles>})
         (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)c.lds);
-    c.partial = c.alloc<double>(mfk::kDotBlocks);
-    c.sc = c.alloc<double>(16);
-    if (!c.partial || !c.sc) return MF_ERR_ALLOC;
     return MF_SUCCESS;
 }
 
@@ -255,7 +371,7 @@ void fill_info(mf_solve_info *info, const MkCtx &c, int status, int it, int repl
     info->replacements = repl;
     info->grid = c.G;
     info->block = 1024;
-    info->layout = 1;  // tile chunks
+    info->layout = c.rows.ok ? (c.mixed && c.rows.narrow ? 3 : 2) : 1;
     info->precision = c.mixed ? MF_PREC_MIXED : MF_PREC_FP64;
     info->relres = bb > 0 ? std::sqrt(std::max(rr, 0.0) / bb) : 0.0;
     info->relres_true = bb > 0 ? std::sqrt(std::max(rt, 0.0) / bb) : std::sqrt(std::max(rt, 0.0));
@@ -266,6 +382,28 @@ void fill_info(mf_solve_info *info, const MkCtx &c, int status, int it, int repl
 
 }  // namespace
 
+// One product of the iteration with its partial sums; returns the number of parts.
+static int mk_cg_product(MkCtx &c, const double *p, const float *p32, const double *r, double *q, double *part)
+{
+    if (!c.rows.ok) {
+        c.spmv(p, p32, q, c.mixed);
+        hipLaunchKernelGGL(mfk::mk_cg_dots, dim3(mfk::kDotBlocks), dim3(1024), 0, c.s, c.n, p, r, q, part, c.sc);
+        return mfk::kDotBlocks;
+    }
+    const RowStreams &R = c.rows;
+    const int ranges = R.P->G, G = std::min(ranges, 2 * c.A->num_cus);
+    auto go = [&](auto k) {
+        hipLaunchKernelGGL(k, dim3(G), dim3(1024), 0, c.s, R.S, R.P->wg_tr, ranges, c.n, p, p32, r, q, part, c.sc);
+    };
+    if (!c.mixed) go(R.rpt == 4 ? mfk::mk_cg_spmv<4, false, false> : R.rpt == 2 ? mfk::mk_cg_spmv<2, false, false>
+                                                                                : mfk::mk_cg_spmv<1, false, false>);
+    else if (R.narrow) go(R.rpt == 4 ? mfk::mk_cg_spmv<4, true, true> : R.rpt == 2 ? mfk::mk_cg_spmv<2, true, true>
+                                                                                   : mfk::mk_cg_spmv<1, true, true>);
+    else go(R.rpt == 4 ? mfk::mk_cg_spmv<4, true, false> : R.rpt == 2 ? mfk::mk_cg_spmv<2, true, false>
+                                                                      : mfk::mk_cg_spmv<1, true, false>);
+    return G;
+}
+
 mf_status cg_multikernel(mf_matrix *A, const double *b, double *x, const mf_solve_options *o, mf_solve_info *info,
                          hipStream_t s)
 {
@@ -273,12 +411,16 @@ mf_status cg_multikernel(mf_matrix *A, const double *b, double *x, const mf_solv
     mf_status st = mk_setup(A, o, s, c);
     if (st != MF_SUCCESS) return st;
     const int n = c.n;
-    double *r = c.alloc<double>(n), *p = c.alloc<double>(n), *q = c.alloc<double>(n);
-    float *p32 = c.mixed ? c.alloc<float>(n) : nullptr;
-    if (!r || !p || !q || (c.mixed && !p32)) return MF_ERR_ALLOC;
+    // vectors from the matrix's workspace, kept from one solve to the next
+    if ((st = A->ws.ensure(n, 1, s)) != MF_SUCCESS) return st;
+    double *r = A->ws.v64, *p = A->ws.p64, *q = A->ws.s64;
+    float *p32 = c.mixed ? A->ws.p32 : nullptr;
+    double *part = c.alloc<double>(4 * (size_t)std::max(mfk::kDotBlocks, 2 * A->num_cus));
+    if (!part) return MF_ERR_ALLOC;
     const dim3 vg = c.vgrid();
     auto t0 = std::chrono::steady_clock::now();
-    // sc: [0] rr [1] pq [2] rr_new [3] bb [4] true rr
+    // sc: [0] r'r [1] iteration [2] state [3] b'b [4] sums of the host's steps
+    if (hipMemsetAsync(c.sc, 0, sizeof(double) * 32, s) != hipSuccess) return MF_ERR_HIP;
     if (o->use_x0) {
         c.spmv(x, nullptr, q, false);
         hipLaunchKernelGGL(mfk::mk_residual, vg, dim3(256), 0, s, b, q, r, (double *)nullptr, (float *)nullptr, n);
@@ -287,48 +429,55 @@ mf_status cg_multikernel(mf_matrix *A, const double *b, double *x, const mf_solv
         hipLaunchKernelGGL(mfk::mk_copy, vg, dim3(256), 0, s, b, r, (float *)nullptr, n);
     }
     hipLaunchKernelGGL(mfk::mk_copy, vg, dim3(256), 0, s, r, p, p32, n);
-    c.dot(r, r, 0);
+    c.dot(r, r, mfk::MKS_RR);
     c.dot(b, b, 3);
     const double bb = c.read(3);
-    double rr = c.read(0), rbase = rr;
+    double rr = c.read(mfk::MKS_RR), rbase = rr;
     int it = 0, repl = 0, status = MF_NOT_CONVERGED;
     const double tol2 = o->tol * o->tol, dl = o->replace_delta > 0 ? o->replace_delta : 1e-3;
     const int max_repl = o->max_replacements > 0 ? o->max_replacements : 64;
     if (bb == 0.0) status = MF_SUCCESS;
+    constexpr int kBatch = 16;
     while (status == MF_NOT_CONVERGED) {
-        if (!o->fixed_iterations) {
-            bool conv = rr <= tol2 * bb;
-            if (c.mixed && repl < max_repl && (conv || rr < dl * dl * rbase)) {
-                c.spmv(x, nullptr, q, false);
-                hipLaunchKernelGGL(mfk::mk_residual, vg, dim3(256), 0, s, b, q, r, p, p32, n);
-                c.dot(r, r, 0);
-                rr = rbase = c.read(0);
-                repl++;
-                conv = rr <= tol2 * bb;
-            }
-            if (conv) {
-                status = MF_SUCCESS;
-                break;
-            }
+        // r'r at or below which the host decides; a tile-mixed solve also looks before the
+        // strict bound dl^2 rbase of a replacement, and at exactly that value goes on
+        const bool may_replace = c.mixed && repl < max_repl;
+        const double below = std::nextafter(dl * dl * rbase, 0.0);
+        const double check2 = o->fixed_iterations ? -1.0 : may_replace ? std::max(tol2 * bb, below) : tol2 * bb;
+        int last = it;
+        for (int i = 0; i < kBatch && last <= o->max_iter; i++, last++) {
+            const int parts = mk_cg_product(c, p, p32, r, q, part);
+            hipLaunchKernelGGL(mfk::mk_cg_update, dim3(mfk::kUpdBlocks), dim3(mfk::kUpdThreads), 0, s, n, parts, part,
+                               check2, last, o->max_iter, x, r, p, p32, q, c.sc);
         }
-        if (it >= o->max_iter) {
+        double h[3];
+        if (hipMemcpyAsync(h, c.sc, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess)
+            return MF_ERR_HIP;
+        rr = h[mfk::MKS_RR];
+        const int state = (int)h[mfk::MKS_STATE];
+        if (state == mfk::MK_RUN) {
+            it = last;
+            continue;
+        }
+        it = (int)h[mfk::MKS_IT];
+        if (state == mfk::MK_BREAK) {
+            status = MF_BREAKDOWN;
+        } else if (state == mfk::MK_MAXIT) {
             status = o->fixed_iterations ? MF_SUCCESS : MF_NOT_CONVERGED;
             break;
+        } else if (!may_replace) {
+            status = MF_SUCCESS;
+        } else {
+            // r = b - A x in binary64, p corrected alike; the iteration is then redone
+            c.spmv(x, nullptr, q, false);
+            hipLaunchKernelGGL(mfk::mk_residual, vg, dim3(256), 0, s, b, q, r, p, p32, n);
+            c.dot(r, r, 4);
+            rr = rbase = c.read(4);
+            repl++;
+            if (rr <= tol2 * bb) status = MF_SUCCESS;
+            else if (hipMemsetAsync(c.sc + mfk::MKS_STATE, 0, sizeof(double), s) != hipSuccess) return MF_ERR_HIP;
         }
-        c.spmv(p, p32, q, c.mixed);
-        c.dot(p, q, 1);
-        hipLaunchKernelGGL(mfk::mk_axpy, vg, dim3(256), 0, s, c.sc, 0, 1, 1.0, p, x, n);
-        hipLaunchKernelGGL(mfk::mk_axpy, vg, dim3(256), 0, s, c.sc, 0, 1, -1.0, q, r, n);
-        c.dot(r, r, 2);
-        hipLaunchKernelGGL(mfk::mk_xpay, vg, dim3(256), 0, s, c.sc, 2, 0, 1u << 1, r, p, p32, n);
-        hipLaunchKernelGGL(mfk::mk_set, dim3(1), dim3(1), 0, s, c.sc, 0, 2);
-        const double pq = c.read(1);
-        if (!(pq != 0.0) || !std::isfinite(pq)) {
-            status = MF_BREAKDOWN;
-            break;
-        }
-        rr = c.read(0);
-        it++;
     }
     // true residual
     c.spmv(x, nullptr, q, false);
