@@ -262,6 +262,13 @@ class TiledMatrix:
         return d
 
     def update_values(self, val):
+        """New values in CSR order: a host array, or a binary64 tensor on the matrix's device."""
+        torch = _torch()
+        if isinstance(val, torch.Tensor) and val.is_cuda:
+            t = _dev_vec(val.detach(), int(self.stats()["nnz"]), torch.device("cuda", self.device))
+            check(L.lib().mf_matrix_update_values_device(self.h, ctypes.c_void_p(t.data_ptr()), _stream_handle()),
+                  "mf_matrix_update_values_device")
+            return
         va = as_f64(val)
         check(L.lib().mf_matrix_update_values(self.h, ptr(va, f64p), _stream_handle()), "mf_matrix_update_values")
 

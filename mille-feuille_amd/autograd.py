@@ -13,8 +13,7 @@ and returns
 Both solves run to the operator's tolerance (default 1e-10 relative residual).  The
 operator keeps a device copy of the values it was last built with: a call with the same
 values compares them on the device and leaves the tiled matrix as it is; changed values
-go through the library's value update (tile classes are a host decision, as in the
-reference's Tile_create).
+go through the library's value update on the device, tile classes included.
 """
 from __future__ import annotations
 
@@ -62,7 +61,7 @@ class SparseOperator:
             return
         self._dvals = t.clone()
         self.version += 1
-        self.A.update_values(t.cpu().numpy())
+        self.A.update_values(self._dvals)
 
     def solve(self, b, transpose=False):
         kw = dict(tol=self.tol, max_iter=self.max_iter, precision=self.precision,

@@ -50,7 +50,7 @@ mf_status upload(void **dst, const void *src, size_t bytes, hipStream_t s)
 
 DeviceLayout::~DeviceLayout() { release(); }
 
-static void free_sell(SellLayout *SL)
+void free_sell(SellLayout *SL)
 {
     if (!SL) return;
     for (int k = 0; k < mfk::kSellStreams; k++) {
@@ -58,6 +58,7 @@ static void free_sell(SellLayout *SL)
         free_dev(SL->idx[k]);
         free_dev(SL->val[k]);
         free_dev(SL->lmask[k]);
+        free_dev(SL->shared[k]);
     }
     for (int w = 0; w < 2; w++) free_dev(SL->win[w]);
     free_dev(SL->perm);
@@ -101,6 +102,23 @@ void DeviceLayout::release()
     src = nullptr;
 }
 
+void class_totals(const TileStruct &ts, const std::vector<uint8_t> &cls, DeviceLayout &L)
+{
+    bool any_lowp = false;
+    for (int c = 0; c < 4; c++) L.tiles_by_class[c] = L.nnz_by_class[c] = 0;
+    for (int64_t t = 0; t < ts.tiles(); t++) {
+        L.tiles_by_class[cls[t]]++;
+        L.nnz_by_class[cls[t]] += ts.tile_off[t + 1] - ts.tile_off[t];
+        if (cls[t] != MF_FP64) any_lowp = true;
+    }
+    L.has_lowp = any_lowp && L.has_copies;
+    // algorithmic bytes of one pass over the value stream (12 B per tile + value + 1 B column)
+    static const double sv[4] = {8, 4, 2, 1};
+    L.alg_bytes_f64 = 12.0 * (double)ts.tiles() + 9.0 * (double)ts.nnz;
+    L.alg_bytes_mixed = 12.0 * (double)ts.tiles();
+    for (int c = 0; c < 4; c++) L.alg_bytes_mixed += (sv[c] + 1.0) * (double)L.nnz_by_class[c];
+}
+
 static mf_status build_layout(const TileStruct &ts, const double *val, const std::vector<uint8_t> &cls,
                               bool keep_mixed, hipStream_t s, DeviceLayout &L)
 {
@@ -139,13 +157,6 @@ static mf_status build_layout(const TileStruct &ts, const double *val, const std
     std::vector<float> v32;
     std::vector<uint16_t> v16;
     std::vector<int8_t> v8;
-    bool any_lowp = false;
-    for (int c = 0; c < 4; c++) L.tiles_by_class[c] = L.nnz_by_class[c] = 0;
-    for (int64_t t = 0; t < T; t++) {
-        L.tiles_by_class[cls[t]]++;
-        L.nnz_by_class[cls[t]] += ts.tile_off[t + 1] - ts.tile_off[t];
-        if (cls[t] != MF_FP64) any_lowp = true;
-    }
     if (keep_mixed) {
         v32.assign(P, 0.f);
         v16.assign(P, 0);
@@ -193,8 +204,8 @@ static mf_status build_layout(const TileStruct &ts, const double *val, const std
     }
     L.max_offset = max_off;
     L.rows_regular = -1;
-    L.has_lowp = any_lowp && !v32.empty();
     L.has_copies = !v32.empty();
+    class_totals(ts, cls, L);
     mf_status st;
     if ((st = upload((void **)&L.eidx, eid.data(), P, s)) != MF_SUCCESS) return st;
     if ((st = upload((void **)&L.v64, v64.data(), sizeof(double) * P, s)) != MF_SUCCESS) return st;
@@ -205,11 +216,6 @@ static mf_status build_layout(const TileStruct &ts, const double *val, const std
         if ((st = upload((void **)&L.v8, v8.data(), P, s)) != MF_SUCCESS) return st;
     }
     if (hipStreamSynchronize(s) != hipSuccess) return MF_ERR_HIP;
-    // algorithmic bytes of one pass over the value stream (12 B per tile + value + 1 B column)
-    static const double sv[4] = {8, 4, 2, 1};
-    L.alg_bytes_f64 = 12.0 * (double)T + 9.0 * (double)ts.nnz;
-    L.alg_bytes_mixed = 12.0 * (double)T;
-    for (int c = 0; c < 4; c++) L.alg_bytes_mixed += (sv[c] + 1.0) * (double)L.nnz_by_class[c];
     L.device_bytes = (double)C * 12 + (double)P * (1 + 8 + 4 + (L.has_copies ? 7 : 0));
     return MF_SUCCESS;
 }
@@ -693,7 +699,8 @@ mf_status ensure_sell(mf_matrix *A, const Partition *Pc, int rpt, bool mixed, hi
     if (mixed && !SL.mixed) mask |= 0xFu;
     if (mask) {
         if (!SL.ordered) choose_order(A, P, SL, allow_perm);
-        mf_status st = SL.permuted ? build_sell(A, P, SL, mask, s) : build_sell_gpu(A, P, SL, mask, s);
+        mf_status st = SL.permuted ? host_values(A, s) : MF_SUCCESS;
+        if (st == MF_SUCCESS) st = SL.permuted ? build_sell(A, P, SL, mask, s) : build_sell_gpu(A, P, SL, mask, s);
         if (st != MF_SUCCESS) {
             free_sell(P.sell);
             P.sell = nullptr;
@@ -839,7 +846,11 @@ extern "C" void mf_matrix_options_default(mf_matrix_options *o)
     o->keep_mixed = 1;
 }
 
-mf_matrix::~mf_matrix() { delete AT; }
+mf_matrix::~mf_matrix()
+{
+    delete AT;
+    for (void *p : {(void *)d_csr, (void *)d_scale, (void *)d_rowptr, (void *)d_moved, (void *)d_cls}) free_dev(p);
+}
 
 extern "C" mf_status mf_matrix_create(int n_rows, int n_cols, const int *rowptr, const int *colidx,
                                       const double *val, const mf_matrix_options *opt, void *stream,
@@ -892,6 +903,7 @@ extern "C" mf_status mf_matrix_update_values(mf_matrix *A, const double *val, vo
     tile_classes(A->ts, A->rowptr.data(), val, A->class_policy, A->cls);
     A->L.release();
     if (A->ts.rows > 0) A->hval.assign(val, val + A->rowptr[A->ts.rows]);
+    A->host_stale = false;
     delete A->AT;  // rebuilt from the new values on the next transposed call
     A->AT = nullptr;
     return build_layout(A->ts, val, A->cls, A->keep_mixed != 0, s, A->L);
@@ -909,6 +921,8 @@ mf_status transposed(mf_matrix *A, hipStream_t s, mf_matrix **out)
         *out = A->AT;
         return MF_SUCCESS;
     }
+    const mf_status hst = host_values(A, s);
+    if (hst != MF_SUCCESS) return hst;
     const TileStruct &ts = A->ts;
     const int m = ts.rows, n = ts.cols;
     if (m > 0 && A->hval.size() < (size_t)A->rowptr[m]) return MF_ERR_UNSUPPORTED;  // created without values

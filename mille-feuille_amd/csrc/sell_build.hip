@@ -230,13 +230,8 @@ struct DevBuf {  // freed on every return
 };
 }  // namespace
 
-mf_status build_sell_gpu(mf_matrix *A, const Partition &P, SellLayout &SL, unsigned mask, hipStream_t s)
+static mfk::SellBuildArgs build_args(const DeviceLayout &L, const Partition &P, const SellLayout &SL)
 {
-    DeviceLayout &L = A->L;
-    const int R = P.G, NW = 16, rpt = SL.rpt, n = L.n_rows;
-    const int64_t slots = (int64_t)R * NW * rpt;
-    mf_status st = L.ensure_tile_order(s);
-    if (st != MF_SUCCESS) return st;
     mfk::SellBuildArgs a;
     a.chunks = L.chunks;
     a.tr_chunk = L.d_tr_chunk;
@@ -246,11 +241,57 @@ mf_status build_sell_gpu(mf_matrix *A, const Partition &P, SellLayout &SL, unsig
     a.v32 = L.v32;
     a.v16 = L.v16;
     a.v8 = L.v8;
-    a.n = n;
-    a.rpt = rpt;
+    a.n = L.n_rows;
+    a.rpt = SL.rpt;
     a.max_off = L.max_offset;
     a.words = (2 * L.max_offset + 1 + 31) / 32;
-    a.slots = slots;
+    a.slots = (long long)P.G * 16 * SL.rpt;
+    return a;
+}
+
+// Column words and values of stream k, whose offsets and flags are in place.
+static void fill_stream(const mfk::SellBuildArgs &a, const SellLayout &SL, int k, hipStream_t s)
+{
+    if (SL.units[k] == 0) return;
+    const int E = mfk::sell_e_host(k, SL.narrow), lgE = E == 2 ? 1 : E == 4 ? 2 : 3;
+    const dim3 grid((unsigned)a.slots), blk(64);
+    int16_t *ix = (int16_t *)SL.idx[k];
+    if (k == 0 || k == mfk::kSellAll64)
+        hipLaunchKernelGGL(mfk::sell_fill_kernel<double>, grid, blk, 0, s, a, k, lgE, SL.soff[k], SL.shared[k], a.v64, ix,
+                           (double *)SL.val[k]);
+    else if (k == 1)
+        hipLaunchKernelGGL(mfk::sell_fill_kernel<float>, grid, blk, 0, s, a, k, lgE, SL.soff[k], SL.shared[k], a.v32, ix,
+                           (float *)SL.val[k]);
+    else if (k == 2)
+        hipLaunchKernelGGL(mfk::sell_fill_kernel<uint16_t>, grid, blk, 0, s, a, k, lgE, SL.soff[k], SL.shared[k], a.v16,
+                           ix, (uint16_t *)SL.val[k]);
+    else
+        hipLaunchKernelGGL(mfk::sell_fill_kernel<int8_t>, grid, blk, 0, s, a, k, lgE, SL.soff[k], SL.shared[k], a.v8, ix,
+                           (int8_t *)SL.val[k]);
+}
+
+mf_status refill_sell(mf_matrix *A, Partition &P, hipStream_t s)
+{
+    if (!P.sell) return MF_SUCCESS;
+    if (P.sell->permuted) {
+        free_sell(P.sell);
+        P.sell = nullptr;
+        return MF_SUCCESS;
+    }
+    const mfk::SellBuildArgs a = build_args(A->L, P, *P.sell);
+    for (int k = 0; k < mfk::kSellStreams; k++)
+        if (P.sell->soff[k]) fill_stream(a, *P.sell, k, s);
+    return hipGetLastError() == hipSuccess ? MF_SUCCESS : MF_ERR_HIP;
+}
+
+mf_status build_sell_gpu(mf_matrix *A, const Partition &P, SellLayout &SL, unsigned mask, hipStream_t s)
+{
+    DeviceLayout &L = A->L;
+    const int R = P.G, NW = 16, rpt = SL.rpt, n = L.n_rows;
+    const int64_t slots = (int64_t)R * NW * rpt;
+    mf_status st = L.ensure_tile_order(s);
+    if (st != MF_SUCCESS) return st;
+    const mfk::SellBuildArgs a = build_args(L, P, SL);
     if (a.words > mfk::kBuildWords) return MF_ERR_TOO_LARGE;
     std::vector<mfk::SellSlot> info((size_t)mfk::kSellStreams * slots);
     DevBuf dinfo;
@@ -347,33 +388,15 @@ mf_status build_sell_gpu(mf_matrix *A, const Partition &P, SellLayout &SL, unsig
         if (u >= INT32_MAX / 64) return MF_ERR_TOO_LARGE;
         SL.units[k] = u;
         const size_t ne = (size_t)u * 64 * E;
-        const int lgE = E == 2 ? 1 : E == 4 ? 2 : 3;
-        DevBuf dshared;
         if ((st = upload((void **)&SL.lmask[k], lm.data(), sizeof(int) * lm.size(), s)) != MF_SUCCESS ||
             (st = upload((void **)&SL.soff[k], soff.data(), sizeof(int) * soff.size(), s)) != MF_SUCCESS ||
-            (st = upload(&dshared.p, shared.data(), shared.size(), s)) != MF_SUCCESS ||
+            (st = upload((void **)&SL.shared[k], shared.data(), shared.size(), s)) != MF_SUCCESS ||
             (st = upload(&SL.idx[k], nullptr, sizeof(int16_t) * ne, s)) != MF_SUCCESS ||
             (st = upload(&SL.val[k], nullptr, ne * mfk::sell_vbytes_host(k), s)) != MF_SUCCESS)
             return st;
         SL.bytes += (double)sizeof(int) * soff.size() + 2.0 * ne + (double)ne * mfk::sell_vbytes_host(k);
-        const dim3 grid((unsigned)slots), blk(64);
-        const uint8_t *ds = (const uint8_t *)dshared.p;
-        int16_t *ix = (int16_t *)SL.idx[k];
-        if (u > 0) {
-            if (k == 0 || k == mfk::kSellAll64)
-                hipLaunchKernelGGL(mfk::sell_fill_kernel<double>, grid, blk, 0, s, a, k, lgE, SL.soff[k], ds, a.v64, ix,
-                                   (double *)SL.val[k]);
-            else if (k == 1)
-                hipLaunchKernelGGL(mfk::sell_fill_kernel<float>, grid, blk, 0, s, a, k, lgE, SL.soff[k], ds, a.v32, ix,
-                                   (float *)SL.val[k]);
-            else if (k == 2)
-                hipLaunchKernelGGL(mfk::sell_fill_kernel<uint16_t>, grid, blk, 0, s, a, k, lgE, SL.soff[k], ds, a.v16, ix,
-                                   (uint16_t *)SL.val[k]);
-            else
-                hipLaunchKernelGGL(mfk::sell_fill_kernel<int8_t>, grid, blk, 0, s, a, k, lgE, SL.soff[k], ds, a.v8, ix,
-                                   (int8_t *)SL.val[k]);
-        }
-        // (the uploads above read these host vectors, and the fill its flags)
+        fill_stream(a, SL, k, s);
+        // (the uploads above read these host vectors)
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) return MF_ERR_HIP;
     }
     for (int w = 0; w < 2; w++) {

@@ -32,6 +32,7 @@ struct SellLayout {
     void *idx[mfk::kSellStreams] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     void *val[mfk::kSellStreams] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     int *lmask[mfk::kSellStreams] = {nullptr, nullptr, nullptr, nullptr, nullptr};  // per wave slot
+    uint8_t *shared[mfk::kSellStreams] = {nullptr, nullptr, nullptr, nullptr, nullptr};  // per slot, rows in order
     int64_t shared_units[mfk::kSellStreams] = {0, 0, 0, 0, 0};  // units of shared-column waves
     int max_wg_units[mfk::kSellStreams] = {0, 0, 0, 0, 0};  // most units one range holds, per stream
     // columns that each range's rows reach, padding included: {first, last + 1} per range, of
@@ -56,6 +57,7 @@ struct Partition {
 };
 
 void free_partition(Partition &P);
+void free_sell(SellLayout *SL);
 
 struct DeviceLayout {
     int n_rows = 0, n_cols = 0, tilem = 0;
@@ -115,6 +117,9 @@ mf_status ensure_sell(mf_matrix *A, const Partition *P, int rpt, bool mixed, hip
 // The streams of `mask` built on the GPU, for ranges that keep their row order
 // (sell_build.hip).
 mf_status build_sell_gpu(mf_matrix *A, const Partition &P, SellLayout &SL, unsigned mask, hipStream_t s);
+// Writes the values of P's streams again from the matrix's value arrays; streams of sorted rows
+// (built on the host) are dropped instead, and rebuilt by the next solve that uses them.
+mf_status refill_sell(mf_matrix *A, Partition &P, hipStream_t s);
 // Padded bytes of one pass over the built class streams (0..3) and over the binary64
 // stream (4) of P's sliced-ELL layout.
 void sell_bytes(const Partition *P, double *class_streams, double *all64);
@@ -211,6 +216,12 @@ struct mf_matrix {
     std::map<long long, int> tuned_grid;  // autotuner cache: key -> workgroups
     int tuned_variant[2] = {0, 0};        // autotuner cache: fp64 / mixed CG variant (0 = default)
     std::vector<double> hval;             // host copy of the CSR values (input positions)
+    // values given on the device (mf_matrix_update_values_device): their copy there, and
+    // whether hval and L.h_ev are older than it (host_values brings them up to date)
+    double *d_csr = nullptr, *d_scale = nullptr;
+    int *d_rowptr = nullptr, *d_moved = nullptr;
+    uint8_t *d_cls = nullptr;             // class per chunk (tile order)
+    bool host_stale = false;
     mf_matrix *AT = nullptr;              // A^T, built on the first transposed call
     mf_matrix() = default;
     mf_matrix(const mf_matrix &) = delete;
@@ -219,6 +230,10 @@ struct mf_matrix {
 };
 
 namespace mf {
+// Tiles, entries and algorithmic bytes per storage class, and whether any is below binary64.
+void class_totals(const TileStruct &ts, const std::vector<uint8_t> &cls, DeviceLayout &L);
+// Brings the host copies of the values up to date with values given on the device.
+mf_status host_values(mf_matrix *A, hipStream_t s);
 // A^T as a tiled matrix of its own (same device, class policy and value copies), built
 // from the host copy of the pattern and values on the first call and kept until the
 // values change.
