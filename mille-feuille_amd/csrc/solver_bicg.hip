@@ -245,10 +245,13 @@ __global__ __launch_bounds__(BLK) void bicg_kernel(BicgArgs a)
             R.refresh();
 #pragma unroll
             for (int k = 0; k < RPT; k++) {
-                if (!R.ok(k)) continue;
-                const double vk = q.get(k, R.loc(k));
-                v.set(k, R.loc(k), vk);
-                d2[0] += a.rhat[R.grow(k)] * vk;
+                // slots past the range hold r = v = 0 (a branch around each row would move
+                // whole register blocks, see cg_core_nb)
+                const bool ok = R.ok(k);
+                const double vk = q.row(k, R.loc(k), ok);
+                if (ok) v.set(k, R.loc(k), vk);
+                const double rh = ok ? a.rhat[R.grow(k)] : 0.0;
+                d2[0] += rh * vk;
                 d2[1] += r[k] * r[k];
             }
             if (!grid_sum<2>(a.gs, d2, epoch, false, wg, scratch)) {
@@ -315,9 +318,9 @@ __global__ __launch_bounds__(BLK) void bicg_kernel(BicgArgs a)
             R.refresh();
 #pragma unroll
             for (int k = 0; k < RPT; k++) {
-                if (!R.ok(k)) continue;
-                const double tk = q.get(k, R.loc(k));
-                const double rh = a.rhat[R.grow(k)];
+                const bool ok = R.ok(k);
+                const double tk = q.row(k, R.loc(k), ok);
+                const double rh = ok ? a.rhat[R.grow(k)] : 0.0;
                 d4[0] += tk * sv[k];
                 d4[1] += tk * tk;
                 d4[2] += rh * sv[k];
