@@ -196,3 +196,23 @@ def test_batch_timeline_and_layout(mf, orc, torch):
     for inf, inf1 in zip(infos, infos1):
         assert abs(inf["iterations"] - inf1["iterations"]) <= 1
     B.close()
+
+
+@pytest.mark.parametrize("sizes", [[40000, 300, 200, 100] + [1000] * 40, [70000, 70000, 9000, 5000, 1], [300] * 3 + [9000]])
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_drained_groups_split(mf, orc, torch, sizes, prec):
+    """Pools of very different lengths on a few workgroups: groups that drained their pool help
+    smaller ones, with and without pools in between, and every system is solved once."""
+    systems = []
+    for i, n in enumerate(sizes):
+        nx = max(1, int(n ** 0.5))
+        rp, ci, va = mf.workloads.poisson2d(nx, max(1, n // nx))
+        b, _ = mf.workloads.rhs_from_solution(rp, ci, va, seed=i)
+        systems.append((rp, ci, va, b))
+    B = mf.Batch([s[:3] for s in systems])
+    b = B.pack([s[3] for s in systems])
+    for grid in (0, 64):
+        x, infos, _ = B.cg(b, tol=1e-9, precision=prec, grid=grid)
+        for (rp, ci, va, bs), xi, inf in zip(systems, B.unpack(x), infos):
+            assert inf["status"] == 0 and orc.true_relres(rp, ci, va, xi, bs) <= 1.2e-9
+    B.close()
