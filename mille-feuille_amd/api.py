@@ -445,4 +445,4 @@ class Batch:
                                           _stream_handle())
         if st not in (L.MF_SUCCESS, 4):
             raise MfError(st, "mf_cg_solve_batched")
-        return x, [infos[i].as_dict() for i in range(self.count)], ms.value
+        return x, L.info_dicts(infos), ms.value
