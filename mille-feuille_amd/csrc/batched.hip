@@ -140,6 +140,16 @@ __device__ __forceinline__ bool batch_worker(const BatchArgs &a, int pool, int W
         part.slot = __builtin_amdgcn_readfirstlane((a.sys_rng0[s] + member) * 16 + (int)(threadIdx.x >> 6));
         part.nb = a.nb;
         part.nb_id = a.sys_rng0[s] + member;
+        part.wlo = part.whi = 0;
+        if constexpr (sell_win(SELL)) {
+            part.wlo = __builtin_amdgcn_readfirstlane(a.S.win[2 * part.nb_id]);
+            part.whi = __builtin_amdgcn_readfirstlane(a.S.win[2 * part.nb_id + 1]);
+            // a group of one never reads the published p: what padding entries reach outside
+            // the rows is zero (the LDS may hold anything)
+            if (SINGLE)
+                for (int i = threadIdx.x; i < part.whi - part.wlo; i += blockDim.x)
+                    if (i + part.wlo < R.row0 || i + part.wlo >= R.row0 + R.nrows) win_put<MIXED>(part, i, 0.0);
+        }
         // variant 4: one group reduction per iteration, p published point to point to the
         // members whose rows gather it (a group of one reduces within the workgroup)
         const CgResult res = cg_core_nb<RPT, MIXED, 1024, U, false, SELL>(part, R, gsy, scratch, q, xs);
@@ -160,14 +170,15 @@ __device__ __forceinline__ bool batch_worker(const BatchArgs &a, int pool, int W
     }
 }
 
-// SELL: 0 tile chunks; 1/2 sliced-ELL streams of the member ranges, wide/narrow profile
+// SELL: 0 tile chunks; 1/2 sliced-ELL streams of the member ranges, wide/narrow profile;
+// + kSellWin: p gathered from an LDS window
 template <int RPT, bool MIXED, int U, int SELL = 0>
 __global__ __launch_bounds__(1024) void batched_cg_kernel(BatchArgs a)
 {
     extern __shared__ double smem[];
     double *scratch = smem;
-    double *q = smem + 64;
-    double *xs = smem + 64 + a.A.rows_cap;
+    double *q = SELL ? nullptr : smem + 64;  // SELL: the SpMV result stays in registers
+    double *xs = SELL ? smem + 64 : smem + 64 + a.A.rows_cap;
     const int b = blockIdx.x;
     int pool = 0;
     while (pool + 1 < a.npools && b >= a.pool_wg0[pool + 1]) pool++;
@@ -458,6 +469,13 @@ static mf_status batch_plan(mf_batch *B, int Gmax, hipStream_t s)
 
 using BatchKernel = void (*)(mfk::BatchArgs);
 
+// Most window columns per row with which a member gathers p from an LDS window: stencil
+// members of 1,000 to 4,000 rows reach 1.1 to 2 columns a row, read once in whole lines where
+// every unit of the SpMV waited for its own gathers, and a group of one workgroup publishes
+// nothing.  Binary64 systems: 7.3 -> 4.5 us an iteration in one workgroup, 10.0 -> 8.1 in
+// two, 10.8 -> 9.9 in sixteen.  Wider windows load more than the gathers they replace.
+constexpr double kBatchWindow = 2.5;
+
 // Kernel for rpt rows per thread and U chunk groups per wave per SpMV batch (U = 0: the
 // register-budget default; the autotuner tries 1 and 2).
 template <bool MIXED, int U>
@@ -472,7 +490,7 @@ static BatchKernel pick_batch_u(int rpt)
     }
 }
 
-// The sliced-ELL kernels (SELL 1 wide, 2 narrow): the chunk-group count does not apply.
+// The sliced-ELL kernels (SELL 1 wide, 2 narrow, + kSellWin): the chunk-group count does not apply.
 template <bool MIXED, int SELL>
 static BatchKernel pick_batch_sell(int rpt)
 {
@@ -485,8 +503,12 @@ static BatchKernel pick_batch_sell(int rpt)
     }
 }
 
-static BatchKernel pick_batch_sell(int rpt, bool mixed, bool narrow)
+static BatchKernel pick_batch_sell(int rpt, bool mixed, bool narrow, bool window)
 {
+    if (window) {
+        if (mixed) return narrow ? pick_batch_sell<true, 2 | mfk::kSellWin>(rpt) : pick_batch_sell<true, 1 | mfk::kSellWin>(rpt);
+        return pick_batch_sell<false, 1 | mfk::kSellWin>(rpt);
+    }
     if (mixed) return narrow ? pick_batch_sell<true, 2>(rpt) : pick_batch_sell<true, 1>(rpt);
     return pick_batch_sell<false, 1>(rpt);
 }
@@ -524,7 +546,7 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
     const int rpt = B->rows_per_wg / 1024;
     BatchKernel k = mixed ? pick_batch<true>(rpt, B->unroll) : pick_batch<false>(rpt, B->unroll);
     if (!k) return MF_ERR_INVALID;
-    const size_t lds = (64 + 2 * (size_t)B->rows_per_wg) * sizeof(double);
+    size_t lds = (64 + 2 * (size_t)B->rows_per_wg) * sizeof(double);
     if (lds > (size_t)A->max_lds) return MF_ERR_TOO_LARGE;
     if (hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return MF_ERR_HIP;
@@ -538,22 +560,36 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
     // no chunk headers, agent-scope gathers.  layout 1 keeps the tile chunks.
     mfk::DevSell dsell;
     memset(&dsell, 0, sizeof(dsell));
+    bool narrow = false;
     if (o.layout != 1 && sell_supported(A, rpt)) {
-        bool narrow = false;
+        bool taken = false;
         if (ensure_sell(A, &B->part, rpt, mixed, s, &dsell, &narrow, false, true) == MF_SUCCESS) {
-            BatchKernel ks = pick_batch_sell(rpt, mixed, narrow);
-            int occ2 = 0;
-            if (ks &&
-                hipFuncSetAttribute((const void *)ks, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) ==
-                    hipSuccess &&
-                hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ2, ks, 1024, lds) == hipSuccess &&
-                B->G <= occ2 * A->num_cus)
+            auto take = [&](BatchKernel ks, size_t bytes) {
+                int occ2 = 0;
+                if (!ks ||
+                    hipFuncSetAttribute((const void *)ks, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) !=
+                        hipSuccess ||
+                    hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ2, ks, 1024, bytes) != hipSuccess ||
+                    B->G > occ2 * A->num_cus)
+                    return false;
                 k = ks;
-            else
-                memset(&dsell, 0, sizeof(dsell));
-        } else {
-            memset(&dsell, 0, sizeof(dsell));
+                lds = bytes;
+                return true;
+            };
+            const SellLayout &SL = *B->part.sell;
+            const size_t at = (64 + (size_t)B->rows_per_wg) * sizeof(double);  // (a multiple of 16)
+            const size_t need = at + (size_t)SL.max_win[mixed] * (mixed ? 4 : 8);
+            // (4 KB left for the kernel's static LDS)
+            if (need + 4096 <= (size_t)A->max_lds && (double)SL.sum_win[mixed] <= kBatchWindow * A->L.n_rows &&
+                take(pick_batch_sell(rpt, mixed, narrow, true), need)) {
+                dsell.win = SL.win[mixed];
+                dsell.win_lds = (int)at;
+                taken = true;
+            } else {
+                taken = take(pick_batch_sell(rpt, mixed, narrow, false), at);
+            }
         }
+        if (!taken) memset(&dsell, 0, sizeof(dsell));
     }
     // records per pool and launched workgroup, publish flags per member range
     if ((st = A->ws.ensure(A->L.n_rows, std::max(B->npools * B->G, B->part.G), s)) != MF_SUCCESS) return st;
@@ -688,7 +724,7 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
             in.block = 1024;
             in.rows_per_thread = rpt;
             // 1 tile chunks, 2/3 sliced-ELL wide/narrow (as mf_solve_info of a single solve)
-            in.layout = a.S.s[mfk::kSellAll64].soff ? (mixed && k == pick_batch_sell(rpt, true, true) ? 3 : 2) : 1;
+            in.layout = a.S.s[mfk::kSellAll64].soff ? (mixed && narrow ? 3 : 2) : 1;
             in.precision = mixed ? MF_PREC_MIXED : MF_PREC_FP64;
         }
     }

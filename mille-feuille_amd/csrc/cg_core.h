@@ -159,7 +159,7 @@ __device__ __forceinline__ void publish_p(const CgPart &a, Rows<RPT, BLK> &R, co
 template <int BLK, bool W32>
 __device__ __forceinline__ void win_halo(const CgPart &a, int row0, int nrows)
 {
-    const i32x4 rs = W32 ? sell_rsrc(a.p32, 4, a.n_sys) : sell_rsrc(a.p64, 8, a.n_sys);
+    const i32x4 rs = W32 ? sell_rsrc(a.p32, 4, a.A.n) : sell_rsrc(a.p64, 8, a.A.n);
     const int below = row0 - a.wlo, halo = a.whi - a.wlo - nrows;  // elements before the rows, in all
     const int t = opaque((int)threadIdx.x);
     constexpr int U = 8;

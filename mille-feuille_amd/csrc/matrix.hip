@@ -625,9 +625,13 @@ static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &
     }
     if (!range_ok) return MF_ERR_TOO_LARGE;
     for (int w = 0; w < 2; w++) {
-        SL.max_win[w] = win[w].empty() ? SL.max_win[w] : 0;
-        for (int r = 0; 2 * (size_t)r < win[w].size(); r++)
+        if (win[w].empty()) continue;
+        SL.max_win[w] = 0;
+        SL.sum_win[w] = 0;
+        for (int r = 0; r < R; r++) {
             SL.max_win[w] = std::max(SL.max_win[w], win[w][2 * r + 1] - win[w][2 * r]);
+            SL.sum_win[w] += win[w][2 * r + 1] - win[w][2 * r];
+        }
     }
     // waves whose column words agree in every lane of every unit
     std::vector<int> lm[mfk::kSellStreams];

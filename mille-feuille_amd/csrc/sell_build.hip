@@ -402,7 +402,11 @@ mf_status build_sell_gpu(mf_matrix *A, const Partition &P, SellLayout &SL, unsig
     for (int w = 0; w < 2; w++) {
         if (win[w].empty()) continue;
         SL.max_win[w] = 0;
-        for (int r = 0; r < R; r++) SL.max_win[w] = std::max(SL.max_win[w], win[w][2 * r + 1] - win[w][2 * r]);
+        SL.sum_win[w] = 0;
+        for (int r = 0; r < R; r++) {
+            SL.max_win[w] = std::max(SL.max_win[w], win[w][2 * r + 1] - win[w][2 * r]);
+            SL.sum_win[w] += win[w][2 * r + 1] - win[w][2 * r];
+        }
         if ((st = upload((void **)&SL.win[w], win[w].data(), sizeof(int) * win[w].size(), s)) != MF_SUCCESS) return st;
     }
     return hipStreamSynchronize(s) == hipSuccess ? MF_SUCCESS : MF_ERR_HIP;

@@ -36,9 +36,11 @@ struct SellLayout {
     int64_t shared_units[mfk::kSellStreams] = {0, 0, 0, 0, 0};  // units of shared-column waves
     int max_wg_units[mfk::kSellStreams] = {0, 0, 0, 0, 0};  // most units one range holds, per stream
     // columns that each range's rows reach, padding included: {first, last + 1} per range, of
-    // the binary64 stream (0) and of the class streams (1), and the widest (sell.h, kSellWin)
+    // the binary64 stream (0) and of the class streams (1), the widest and all together
+    // (sell.h, kSellWin)
     int *win[2] = {nullptr, nullptr};
     int max_win[2] = {0, 0};
+    int64_t sum_win[2] = {0, 0};
     double bytes = 0;               // device bytes of the built streams
 };
 
