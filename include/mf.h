@@ -261,8 +261,10 @@ typedef struct mf_solve_info {
     int variant;
     int precision;          /* arithmetic used: MF_PREC_MIXED, or MF_PREC_FP64 -- also for a
                                tile-mixed request when the matrix has no lower-precision tiles,
-                               or (layout default) when its class streams would move as many
-                               bytes as the binary64 stream */
+                               or (layout default) when binary64 arithmetic is the faster: the
+                               class streams would move as many bytes as the binary64 stream,
+                               the binary64 stream of a CG fits the workgroups' LDS, or the
+                               class streams of a batch hold nearly as many units */
 } mf_solve_info;
 
 void mf_solve_options_default(mf_solve_options *o);

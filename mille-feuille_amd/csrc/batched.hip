@@ -469,6 +469,13 @@ static mf_status batch_plan(mf_batch *B, int Gmax, hipStream_t s)
 
 using BatchKernel = void (*)(mfk::BatchArgs);
 
+// Most units of the binary64 stream per unit of the class streams with which a tile-mixed
+// batch runs binary64 arithmetic.  Its SpMV waits for units, not bytes, and class streams
+// start their pipelines one after another: shifted Laplacians (3 units of two class streams
+// for 3 or 4) take 9.9 us an iteration in binary64 and 11.7 tile-mixed in groups of sixteen,
+// 4.5 and 5.5 in groups of one, and need no residual replacements.
+constexpr double kBatchUnits64 = 1.5;
+
 // Most window columns per row with which a member gathers p from an LDS window: stencil
 // members of 1,000 to 4,000 rows reach 1.1 to 2 columns a row, read once in whole lines where
 // every unit of the SpMV waited for its own gathers, and a group of one workgroup publishes
@@ -542,7 +549,7 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
     // every launch starts from x = 0 (the reset clears x with the publish buffers), and
     // the batched core has neither the transposed streams nor the dynamic classes
     if (o.use_x0 || o.transpose || o.dynamic_precision) return MF_ERR_UNSUPPORTED;
-    const bool mixed = o.precision == MF_PREC_MIXED && A->L.has_lowp;
+    bool mixed = o.precision == MF_PREC_MIXED && A->L.has_lowp;
     const int rpt = B->rows_per_wg / 1024;
     BatchKernel k = mixed ? pick_batch<true>(rpt, B->unroll) : pick_batch<false>(rpt, B->unroll);
     if (!k) return MF_ERR_INVALID;
@@ -577,6 +584,10 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
                 return true;
             };
             const SellLayout &SL = *B->part.sell;
+            const bool asked = mixed;
+            int64_t low = 0;
+            for (int c = 0; c < mfk::kSellAll64; c++) low += SL.units[c];
+            if (o.layout == 0 && (double)SL.units[mfk::kSellAll64] <= kBatchUnits64 * (double)low) mixed = false;
             const size_t at = (64 + (size_t)B->rows_per_wg) * sizeof(double);  // (a multiple of 16)
             const size_t need = at + (size_t)SL.max_win[mixed] * (mixed ? 4 : 8);
             // (4 KB left for the kernel's static LDS)
@@ -588,6 +599,7 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
             } else {
                 taken = take(pick_batch_sell(rpt, mixed, narrow, false), at);
             }
+            if (!taken) mixed = asked;
         }
         if (!taken) memset(&dsell, 0, sizeof(dsell));
     }

@@ -682,6 +682,22 @@ void sell_bytes(const Partition *P, double *class_streams, double *all64)
     }
 }
 
+// LDS bytes of one range's copy of the value streams a solve reads (class streams 0..3 for
+// tile-mixed arithmetic, the binary64 stream otherwise), each region 16-byte aligned.
+size_t sell_lds_bytes(const SellLayout &SL, bool mixed_arith, size_t offsets[mfk::kSellStreams], size_t base)
+{
+    size_t off = (base + 15) / 16 * 16;
+    for (int k = 0; k < mfk::kSellStreams; k++) {
+        offsets[k] = (size_t)-1;
+        const bool used = mixed_arith ? k < mfk::kSellAll64 : k == mfk::kSellAll64;
+        if (!used || SL.max_wg_units[k] == 0) continue;
+        offsets[k] = off;
+        off += (size_t)SL.max_wg_units[k] * 64 * mfk::sell_e_host(k, SL.narrow) * mfk::sell_vbytes_host(k);
+        off = (off + 15) / 16 * 16;
+    }
+    return off;
+}
+
 mf_status ensure_sell(mf_matrix *A, const Partition *Pc, int rpt, bool mixed, hipStream_t s, mfk::DevSell *out,
                       bool *narrow, bool allow_perm, bool build)
 {

@@ -153,22 +153,6 @@ static CgKernel cg_sell_win_kernel_for(int rpt, bool mixed, bool narrow, bool pe
                   : pick_cg<4, true, false, false, 1 | mfk::kSellWin>(rpt);
 }
 
-// LDS bytes of one range's copy of the value streams a solve reads (class streams 0..3 for
-// tile-mixed arithmetic, the binary64 stream otherwise), each region 16-byte aligned.
-static size_t sell_lds_bytes(const SellLayout &SL, bool mixed_arith, size_t offsets[mfk::kSellStreams], size_t base)
-{
-    size_t off = (base + 15) / 16 * 16;
-    for (int k = 0; k < mfk::kSellStreams; k++) {
-        offsets[k] = (size_t)-1;
-        const bool used = mixed_arith ? k < mfk::kSellAll64 : k == mfk::kSellAll64;
-        if (!used || SL.max_wg_units[k] == 0) continue;
-        offsets[k] = off;
-        off += (size_t)SL.max_wg_units[k] * 64 * mfk::sell_e_host(k, SL.narrow) * mfk::sell_vbytes_host(k);
-        off = (off + 15) / 16 * 16;
-    }
-    return off;
-}
-
 static CgKernel cg_sell_kernel_for(int rpt, int var, bool mixed, bool narrow, bool perm)
 {
     if (perm) {
@@ -294,8 +278,9 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     // iteration against 6.2 on tile chunks); tile chunks for the other all-FP64 solves,
     // whose streams are bandwidth-bound and where the chunks carry less padding.  layout
     // 1 / 2 force chunks / sliced-ELL.
-    const bool fp64_small = o->layout == 0 && !mixed && !dyn && o->value_cache == 0 && !sparse_tiles(A) &&
-                            (double)A->L.nnz * 8.0 * 1.5 / G + (double)lds_x + 4096.0 <= (double)A->max_lds;
+    // (1.2: a 7-point row of 8 slots, and the ragged last slices)
+    const bool small64 = (double)A->L.nnz * 8.0 * 1.2 / G + (double)lds_x + 4096.0 <= (double)A->max_lds;
+    const bool fp64_small = o->layout == 0 && !mixed && !dyn && o->value_cache == 0 && !sparse_tiles(A) && small64;
     const bool want_sell = o->layout == 2 || (o->layout == 0 && (mixed || sparse_tiles(A) || fp64_small));
     bool sell = want_sell && !dyn && sell_supported(A, rpt) && lds_x <= (size_t)A->max_lds;
     size_t lds = sell ? lds_x : (64 + 2 * (size_t)std::max(P->rows_cap, 1)) * sizeof(double);
@@ -313,14 +298,26 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     mfk::DevSell dsell;
     memset(&dsell, 0, sizeof(dsell));
     bool narrow = false;
-    if (sell && (st = ensure_sell(A, P, rpt, mixed, s, &dsell, &narrow,
-                                  cg_perm_supported(rpt, var) && A->L.n_rows > kPermMinRows * G, !ext)) != MF_SUCCESS)
-        return st;
+    const bool perm_ok = cg_perm_supported(rpt, var) && A->L.n_rows > kPermMinRows * G;
+    // A tile-mixed solve whose binary64 stream fits the workgroups' LDS runs binary64
+    // arithmetic on it (reported in info->precision): with the values on chip the SpMV waits
+    // for units, not bytes, class streams start their pipelines one after another, and no
+    // residual is replaced.  Laplacians, tile-mixed / binary64, us per iteration: 64^3 shifted
+    // 8.4 / 7.0, 40 x 41 x 42 shifted 8.1 / 6.9, 300 x 301 shifted 7.6 / 6.8, 50^3 (one class)
+    // 7.1 / 6.9.  The arithmetic does not depend on value_cache, so both settings agree.
+    bool mixed_arith = mixed;
+    if (sell && mixed && var == 4 && o->layout == 0 && small64) {
+        if ((st = ensure_sell(A, P, rpt, false, s, &dsell, &narrow, perm_ok, !ext)) != MF_SUCCESS) return st;
+        size_t offs[mfk::kSellStreams];
+        if (!dsell.perm && cg_sell_lds_kernel_for(rpt, false, narrow) &&
+            sell_lds_bytes(*P->sell, false, offs, lds_x) + 4096 <= (size_t)A->max_lds)
+            mixed_arith = false;
+    }
+    if (sell && (st = ensure_sell(A, P, rpt, mixed_arith, s, &dsell, &narrow, perm_ok, !ext)) != MF_SUCCESS) return st;
     // Tile-mixed solve whose class streams would move about as many bytes as the binary64
     // stream (rows spread over classes pad each class stream): binary64 arithmetic on the
     // binary64 stream is then as fast and exact; reported in info->precision.
-    bool mixed_arith = mixed;
-    if (sell && mixed && o->layout == 0) {
+    if (sell && mixed_arith && o->layout == 0) {
         double bc = 0, b64 = 0;
         sell_bytes(P, &bc, &b64);
         if (bc >= 0.95 * b64) mixed_arith = false;

@@ -125,6 +125,7 @@ mf_status refill_sell(mf_matrix *A, Partition &P, hipStream_t s);
 // Padded bytes of one pass over the built class streams (0..3) and over the binary64
 // stream (4) of P's sliced-ELL layout.
 void sell_bytes(const Partition *P, double *class_streams, double *all64);
+size_t sell_lds_bytes(const SellLayout &SL, bool mixed_arith, size_t offsets[mfk::kSellStreams], size_t base);
 
 
 // Sliced-ELL streams over ranges of 1024 rpt consecutive rows for products launched by
