@@ -57,3 +57,19 @@ def test_batched_members(mf, orc, torch, rows_per_wg, prec, layout, shift, arith
                 ref = orc.cg(rp, ci, va, bs, tol=1e-10)
                 assert abs(inf["iterations"] - ref["iterations"]) <= max(1, 0.02 * ref["iterations"])
     B.close()
+
+
+@pytest.mark.parametrize("nx", [3, 10, 31, 40, 63, 70])
+def test_bicgstab_stream_in_lds(mf, orc, torch, nx):
+    """All-FP64 BiCGSTAB with its binary64 stream in LDS: the words and the order of the sums
+    are those of the stream in memory, so the bits agree; also transposed."""
+    rp, ci, va = mf.workloads.convdiff3d(nx)
+    b, _ = mf.workloads.rhs_from_solution(rp, ci, va, seed=2)
+    A = mf.TiledMatrix(rp, ci, va)
+    for transpose in (False, True):
+        x, info = A.bicgstab(b, tol=1e-10, transpose=transpose)
+        y, mem = A.bicgstab(b, tol=1e-10, transpose=transpose, value_cache=False)
+        assert info["status"] == mem["status"] == 0 and mem["layout"] == 2
+        assert info["layout"] == (6 if nx <= 63 else info["layout"])
+        assert info["iterations"] == mem["iterations"] and np.array_equal(x.cpu().numpy(), y.cpu().numpy())
+    A.close()
