@@ -225,7 +225,7 @@ __device__ __forceinline__ bool replace_residual(const CgPart &a, Rows<RPT, BLK>
 // a.x; every member returns the same CgResult.
 template <int RPT, int VAR, bool MIXED, int BLK, class Sync, int U = spmv_unroll<RPT, 2>(), bool XREG = false,
           bool DYN = false, int SELL = 0>
-__device__ __forceinline__ CgResult cg_core(const CgPart &a, Rows<RPT, BLK> &R, Sync &sy, double *scratch, double *q_lds,
+__device__ CgResult cg_core(const CgPart &a, Rows<RPT, BLK> &R, Sync &sy, double *scratch, double *q_lds,
                             double *xs_lds)
 {
     XVec<RPT, XREG> xs;
@@ -966,9 +966,14 @@ __global__ __launch_bounds__(BLK) void cg_kernel(CgArgs a)
     else if constexpr (VAR == 3)
         res = cg_core_pipelined<RPT, MIXED, BLK, GridOps, spmv_unroll<RPT, XREG ? 6 : 5>(), XREG, SELL>(
             part, R, sy, scratch, q, xs);
+    else if constexpr (DYN)
+        // not forced inline: inlined into the kernel the core under dynamic classes spills 500
+        // VGPRs at 8 rows per thread (3D Poisson 128^3 45.0 ms instead of 36.8); the other
+        // variants need it (variant 1 on class streams 17.9 -> 7.6 ms)
+        res = cg_core<RPT, VAR, MIXED, BLK, GridOps, spmv_unroll<RPT, 3>(), XREG, DYN, SELL>(part, R, sy, scratch, q, xs);
     else
-        res = cg_core<RPT, VAR, MIXED, BLK, GridOps, spmv_unroll<RPT, (XREG || DYN) ? 3 : 2>(), XREG, DYN, SELL>(
-            part, R, sy, scratch, q, xs);
+        [[clang::always_inline]] res = cg_core<RPT, VAR, MIXED, BLK, GridOps, spmv_unroll<RPT, XREG ? 3 : 2>(), XREG, DYN,
+                                               SELL>(part, R, sy, scratch, q, xs);
     if (wg == 0 && threadIdx.x == 0) {
         a.info[0] = (double)res.it;
         a.info[1] = res.rr;
