@@ -966,14 +966,15 @@ __global__ __launch_bounds__(BLK) void cg_kernel(CgArgs a)
     else if constexpr (VAR == 3)
         res = cg_core_pipelined<RPT, MIXED, BLK, GridOps, spmv_unroll<RPT, XREG ? 6 : 5>(), XREG, SELL>(
             part, R, sy, scratch, q, xs);
-    else if constexpr (DYN)
+    else if constexpr (DYN && RPT == 8)
         // not forced inline: inlined into the kernel the core under dynamic classes spills 500
-        // VGPRs at 8 rows per thread (3D Poisson 128^3 45.0 ms instead of 36.8); the other
-        // variants need it (variant 1 on class streams 17.9 -> 7.6 ms)
+        // VGPRs at 8 rows per thread (3D Poisson 128^3 45.0 ms, 35.9 out of line); fewer rows
+        // need it (48^3 2.8 ms, 4.6 out of line), and so do the other variants (variant 1 on
+        // class streams 17.9 -> 7.6 ms)
         res = cg_core<RPT, VAR, MIXED, BLK, GridOps, spmv_unroll<RPT, 3>(), XREG, DYN, SELL>(part, R, sy, scratch, q, xs);
     else
-        [[clang::always_inline]] res = cg_core<RPT, VAR, MIXED, BLK, GridOps, spmv_unroll<RPT, XREG ? 3 : 2>(), XREG, DYN,
-                                               SELL>(part, R, sy, scratch, q, xs);
+        [[clang::always_inline]] res = cg_core<RPT, VAR, MIXED, BLK, GridOps, spmv_unroll<RPT, (XREG || DYN) ? 3 : 2>(), XREG,
+                                               DYN, SELL>(part, R, sy, scratch, q, xs);
     if (wg == 0 && threadIdx.x == 0) {
         a.info[0] = (double)res.it;
         a.info[1] = res.rr;
