@@ -280,8 +280,8 @@ mf_status mf_matrix_get_stats(const mf_matrix *A, mf_matrix_stats *st);
 /* Overwrite the values (same pattern, CSR order; host array), e.g. for finite
  * differences: storage classes and value streams are rebuilt, the tiles are kept. */
 mf_status mf_matrix_update_values(mf_matrix *A, const double *val, void *stream);
-/* The same from a device array (CSR order, indexed like val above): classes, value arrays and
- * streams are renewed on the device. */
+/* The same from a device array (CSR order, indexed like val above, so rowptr[n_rows] values when
+ * rowptr[0] > 0): classes, value arrays and streams are renewed on the device. */
 mf_status mf_matrix_update_values_device(mf_matrix *A, const double *d_val, void *stream);
 /* d_out[k] = scale * d_u[row(k)] * d_v[col(k)] for every stored entry k, written in the
  * CSR order of the input (the value gradient -lambda_i x_j of an adjoint solve). */

@@ -228,6 +228,9 @@ class TiledMatrix:
     def __init__(self, rowptr, colidx, val, n_cols=None, class_policy="lossless", device=0, keep_mixed=True):
         rp, ci, va = as_i32(rowptr), as_i32(colidx), as_f64(val)
         self.n = int(rp.size - 1)
+        # lengths of a value vector: the rows' CSR positions (from 0, also when rowptr[0] > 0),
+        # or the array given here, which may go on after them
+        self._val_lengths = (int(rp[-1]), int(va.size))
         self.n_cols = int(n_cols if n_cols is not None else self.n)
         self.device = int(device)
         mo = L.MatrixOptions()
@@ -262,10 +265,13 @@ class TiledMatrix:
         return d
 
     def update_values(self, val):
-        """New values in CSR order: a host array, or a binary64 tensor on the matrix's device."""
+        """New values in CSR order: a host array, or a binary64 tensor on the matrix's device.
+        Both are indexed by CSR position, so they reach rowptr[n]."""
         torch = _torch()
         if isinstance(val, torch.Tensor) and val.is_cuda:
-            t = _dev_vec(val.detach(), int(self.stats()["nnz"]), torch.device("cuda", self.device))
+            if val.numel() not in self._val_lengths or val.numel() < self._val_lengths[0]:
+                raise ValueError(f"{val.numel()} values, expected {self._val_lengths[0]}")
+            t = _dev_vec(val.detach(), val.numel(), torch.device("cuda", self.device))
             check(L.lib().mf_matrix_update_values_device(self.h, ctypes.c_void_p(t.data_ptr()), _stream_handle()),
                   "mf_matrix_update_values_device")
             return
