@@ -55,10 +55,8 @@ struct BatchArgs {
 };
 
 // Before each batched launch: records, abort flag and queues, and -- for the sliced-ELL
-// kernels -- the publish buffers and x over every row of the block-diagonal matrix.  A
-// sliced-ELL row's zero-valued padding entries gather p (and, in residual checks, x) at
-// rows of other systems or between systems; those must hold finite values, since
-// 0 * NaN is NaN (every solve starts from x = 0, and writes x for its own rows).
+// kernels -- the publish buffers and x over every row of the block-diagonal matrix (every
+// solve starts from x = 0 and writes x for its own rows; the rows between systems stay 0).
 __global__ void batch_reset_kernel(unsigned long long *recs, long long n, unsigned *ctl, unsigned *queue, int npools,
                                    unsigned *flags, long long nflags, double *p64, float *p32, double *x,
                                    long long nrows)
@@ -109,21 +107,26 @@ __device__ __forceinline__ bool batch_worker(const BatchArgs &a, int pool, int W
         }
         if (idx >= nsys) return true;
         const unsigned long long t_start = __builtin_amdgcn_s_memrealtime();
-        const int s = a.order[a.pool_sys0[pool] + idx];
+        const int s = __builtin_amdgcn_readfirstlane(a.order[a.pool_sys0[pool] + idx]);
         const int t0 = a.sys_tr[s], t1 = a.sys_tr[s + 1];
+        // Sliced-ELL: rows and columns count from the system's first row.  Zero-valued padding
+        // entries name columns outside the system, whose p may hold a NaN or an infinity (and
+        // 0 * NaN is NaN); with the vectors' bounds at the system's rows those gathers read 0.
+        // (Tile chunks hold absolute rows and columns, and no padding.)
+        const int c0 = SELL ? t0 * kTile : 0;
         const int mt0 = t0 + (int)((long long)(t1 - t0) * member / W);
         const int mt1 = t0 + (int)((long long)(t1 - t0) * (member + 1) / W);
         Rows<RPT, 1024> R;
-        R.row0 = mt0 * kTile;
-        R.nrows = max(0, min(mt1 * kTile, t0 * kTile + a.sys_rows[s]) - R.row0);
+        R.row0 = mt0 * kTile - c0;
+        R.nrows = max(0, min(mt1 * kTile, t0 * kTile + a.sys_rows[s]) - mt0 * kTile);
         R.refresh();
         CgPart part;
         part.A = a.A;
         part.cr = a.A.wg_chunk + 4 * (size_t)(a.sys_rng0[s] + member);
-        part.b = a.b;
-        part.x = a.x;
-        part.p64 = a.p64;
-        part.p32 = a.p32;
+        part.b = a.b + c0;
+        part.x = a.x + c0;
+        part.p64 = a.p64 + c0;
+        part.p32 = a.p32 + c0;
         part.tol2 = a.tol2;
         part.delta2 = a.delta2;
         part.maxit = a.maxit;
@@ -136,14 +139,19 @@ __device__ __forceinline__ bool batch_worker(const BatchArgs &a, int pool, int W
         part.dyn_mode = 0;
         part.n_sys = a.sys_rows[s];
         part.S = a.S;
+        if constexpr (SELL != 0) {
+            part.A.n = a.sys_rows[s];
+#pragma unroll
+            for (int k = 0; k < kSellStreams; k++) part.S.s[k].xmax = a.sys_rows[s] - 1;
+        }
         // this wave's slot in the member range's streams
         part.slot = __builtin_amdgcn_readfirstlane((a.sys_rng0[s] + member) * 16 + (int)(threadIdx.x >> 6));
         part.nb = a.nb;
         part.nb_id = a.sys_rng0[s] + member;
         part.wlo = part.whi = 0;
         if constexpr (sell_win(SELL)) {
-            part.wlo = __builtin_amdgcn_readfirstlane(a.S.win[2 * part.nb_id]);
-            part.whi = __builtin_amdgcn_readfirstlane(a.S.win[2 * part.nb_id + 1]);
+            part.wlo = __builtin_amdgcn_readfirstlane(a.S.win[2 * part.nb_id]) - c0;
+            part.whi = __builtin_amdgcn_readfirstlane(a.S.win[2 * part.nb_id + 1]) - c0;
             // a group of one never reads the published p: what padding entries reach outside
             // the rows is zero (the LDS may hold anything)
             if (SINGLE)
