@@ -575,10 +575,10 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
     // no chunk headers, agent-scope gathers.  layout 1 keeps the tile chunks.
     mfk::DevSell dsell;
     memset(&dsell, 0, sizeof(dsell));
-    bool narrow = false;
+    const SellLayout *layout = nullptr;
     if (o.layout != 1 && sell_supported(A, rpt)) {
         bool taken = false;
-        if (ensure_sell(A, &B->part, rpt, mixed, s, &dsell, &narrow, false, true) == MF_SUCCESS) {
+        if (ensure_sell(A, &B->part, rpt, mixed, s, &dsell, &layout, false, true) == MF_SUCCESS) {
             auto take = [&](BatchKernel ks, size_t bytes) {
                 int occ2 = 0;
                 if (!ks ||
@@ -591,7 +591,8 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
                 lds = bytes;
                 return true;
             };
-            const SellLayout &SL = *B->part.sell;
+            const SellLayout &SL = *layout;
+            const bool narrow = SL.narrow;
             const bool asked = mixed;
             int64_t low = 0;
             for (int c = 0; c < mfk::kSellAll64; c++) low += SL.units[c];
@@ -744,7 +745,7 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
             in.block = 1024;
             in.rows_per_thread = rpt;
             // 1 tile chunks, 2/3 sliced-ELL wide/narrow (as mf_solve_info of a single solve)
-            in.layout = a.S.s[mfk::kSellAll64].soff ? (mixed && narrow ? 3 : 2) : 1;
+            in.layout = a.S.s[mfk::kSellAll64].soff ? (mixed && layout->narrow ? 3 : 2) : 1;
             in.precision = mixed ? MF_PREC_MIXED : MF_PREC_FP64;
         }
     }

@@ -70,13 +70,14 @@ void free_partition(Partition &P)
     free_dev(P.wg_tr);
     free_dev(P.wg_chunk);
     free_dev(P.chunks);
-    free_sell(P.sell);
+    for (SellLayout *SL : P.sell) free_sell(SL);
     free_dev(P.dep_ptr);
     free_dev(P.dep_idx);
     P.wg_tr = nullptr;
     P.wg_chunk = nullptr;
     P.chunks = nullptr;
-    P.sell = nullptr;
+    P.sell[0] = P.sell[1] = nullptr;
+    P.sort_pays = -1;
     P.dep_ptr = P.dep_idx = nullptr;
 }
 
@@ -382,15 +383,13 @@ static void range_rows(const TileStruct &ts, int tr0, int tr1, int r0, int nr, s
                 ent[at[bi * kTile + ts.lrow[e] - r0]++] = {e, t};
 }
 
-// Decides whether the ranges' rows are sorted by length (longest first, stably) for the
-// streams of partition P: when that cuts the padded binary64 stream by 10 % or more.  Fills
-// SL.permuted and, when sorted, SL.h_perm.
-static void choose_order(const mf_matrix *A, const Partition &P, SellLayout &SL, bool allow_perm)
+// Whether sorting the ranges' rows by length (longest first, stably) pays for the streams of
+// partition P: when it cuts the padded binary64 stream by 10 % or more.  Then *out is a layout
+// (no streams yet) that holds the permutation.
+static bool choose_order(const mf_matrix *A, const Partition &P, int rpt, SellLayout **out)
 {
-    SL.ordered = true;
-    SL.permuted = false;
-    if (!allow_perm || A->rowptr.empty()) return;
-    const int R = P.G, LOC = 1024 * SL.rpt, n = A->L.n_rows;
+    if (A->rowptr.empty()) return false;
+    const int R = P.G, LOC = 1024 * rpt, n = A->L.n_rows;
     const int *rp = A->rowptr.data();
     std::vector<double> pad_id(R, 0.0), pad_sorted(R, 0.0);
     std::vector<std::vector<int>> sorted(R);
@@ -418,14 +417,19 @@ static void choose_order(const mf_matrix *A, const Partition &P, SellLayout &SL,
         pi += pad_id[r];
         ps += pad_sorted[r];
     }
-    SL.permuted = ps < 0.9 * pi;
-    if (!SL.permuted) return;
-    SL.h_perm.assign((size_t)R * LOC, 0);
+    if (!(ps < 0.9 * pi)) return false;
+    SellLayout *SL = new SellLayout();
+    SL->rpt = rpt;
+    SL->permuted = true;
+    SL->h_perm.assign((size_t)R * LOC, 0);
     for (int r = 0; r < R; r++) {
         const int r0 = P.h_tr[r] * kTile, nr = std::max(0, std::min(P.h_tr[r + 1] * kTile, n) - r0);
-        int *pr = SL.h_perm.data() + (size_t)r * LOC;
+        int *pr = SL->h_perm.data() + (size_t)r * LOC;
         for (int i = 0; i < LOC; i++) pr[i] = i < nr ? sorted[r][i] : std::max(0, nr - 1);
     }
+    free_sell(*out);
+    *out = SL;
+    return true;
 }
 
 // Builds the sliced-ELL streams in `mask` (bit s: stream s) on the host for partition P,
@@ -670,13 +674,11 @@ static mf_status build_sell(const mf_matrix *A, const Partition &P, SellLayout &
     return st;
 }
 
-void sell_bytes(const Partition *P, double *class_streams, double *all64)
+void sell_bytes(const SellLayout &SL, double *class_streams, double *all64)
 {
     *class_streams = *all64 = 0.0;
-    const SellLayout *SL = P->sell;
-    if (!SL) return;
     for (int k = 0; k < mfk::kSellStreams; k++) {
-        const double b = (double)SL->units[k] * 64 * mfk::sell_e_host(k, SL->narrow) * (2 + mfk::sell_vbytes_host(k));
+        const double b = (double)SL.units[k] * 64 * mfk::sell_e_host(k, SL.narrow) * (2 + mfk::sell_vbytes_host(k));
         if (k == mfk::kSellAll64) *all64 += b;
         else *class_streams += b;
     }
@@ -699,31 +701,42 @@ size_t sell_lds_bytes(const SellLayout &SL, bool mixed_arith, size_t offsets[mfk
 }
 
 mf_status ensure_sell(mf_matrix *A, const Partition *Pc, int rpt, bool mixed, hipStream_t s, mfk::DevSell *out,
-                      bool *narrow, bool allow_perm, bool build)
+                      const SellLayout **layout, bool allow_perm, bool build)
 {
     // the sliced-ELL streams are a cache of the partition, rebuilt with it
     Partition &P = const_cast<Partition &>(*Pc);
-    if (!build && (!P.sell || P.sell->rpt != rpt || !P.sell->soff[mfk::kSellAll64] || (mixed && !P.sell->mixed)))
+    for (SellLayout *&SL : P.sell)
+        if (build && SL && SL->rpt != rpt) {
+            free_sell(SL);
+            SL = nullptr;
+            P.sort_pays = -1;
+        }
+    if (build && allow_perm && P.sort_pays < 0) P.sort_pays = choose_order(A, P, rpt, &P.sell[1]) ? 1 : 0;
+    if (!allow_perm && rpt >= 4 && P.sell[1] && !P.sell[0]) {
+        // no second copy of a large range's streams for a caller without kernels for sorted
+        // rows: it sees the permutation and keeps the tile chunks
+        out->perm = P.sell[1]->perm;
+        *layout = P.sell[1];
+        return MF_SUCCESS;
+    }
+    SellLayout *&cache = P.sell[allow_perm && P.sort_pays == 1 ? 1 : 0];
+    if (!build && (!cache || cache->rpt != rpt || !cache->soff[mfk::kSellAll64] || (mixed && !cache->mixed)))
         return MF_ERR_UNSUPPORTED;
-    if (P.sell && P.sell->rpt != rpt) {
-        free_sell(P.sell);
-        P.sell = nullptr;
+    if (!cache) {
+        cache = new SellLayout();
+        cache->rpt = rpt;
     }
-    if (!P.sell) {
-        P.sell = new SellLayout();
-        P.sell->rpt = rpt;
-    }
-    SellLayout &SL = *P.sell;
+    SellLayout &SL = *cache;
     unsigned mask = 0;
     if (!SL.soff[mfk::kSellAll64]) mask |= 1u << mfk::kSellAll64;
     if (mixed && !SL.mixed) mask |= 0xFu;
     if (mask) {
-        if (!SL.ordered) choose_order(A, P, SL, allow_perm);
         mf_status st = SL.permuted ? host_values(A, s) : MF_SUCCESS;
         if (st == MF_SUCCESS) st = SL.permuted ? build_sell(A, P, SL, mask, s) : build_sell_gpu(A, P, SL, mask, s);
         if (st != MF_SUCCESS) {
-            free_sell(P.sell);
-            P.sell = nullptr;
+            if (SL.permuted) P.sort_pays = -1;
+            free_sell(cache);
+            cache = nullptr;
             return st;
         }
         if (mask & 0xFu) SL.mixed = true;
@@ -737,7 +750,7 @@ mf_status ensure_sell(mf_matrix *A, const Partition *Pc, int rpt, bool mixed, hi
         out->s[k].lds = -1;  // the launcher decides which streams a kernel holds in LDS
     }
     out->perm = SL.perm;
-    *narrow = SL.narrow;
+    *layout = &SL;
     return MF_SUCCESS;
 }
 

@@ -272,15 +272,14 @@ static void fill_stream(const mfk::SellBuildArgs &a, const SellLayout &SL, int k
 
 mf_status refill_sell(mf_matrix *A, Partition &P, hipStream_t s)
 {
-    if (!P.sell) return MF_SUCCESS;
-    if (P.sell->permuted) {
-        free_sell(P.sell);
-        P.sell = nullptr;
-        return MF_SUCCESS;
-    }
-    const mfk::SellBuildArgs a = build_args(A->L, P, *P.sell);
+    free_sell(P.sell[1]);
+    P.sell[1] = nullptr;
+    P.sort_pays = -1;
+    if (!P.sell[0]) return MF_SUCCESS;
+    const SellLayout &SL = *P.sell[0];
+    const mfk::SellBuildArgs a = build_args(A->L, P, SL);
     for (int k = 0; k < mfk::kSellStreams; k++)
-        if (P.sell->soff[k]) fill_stream(a, *P.sell, k, s);
+        if (SL.soff[k]) fill_stream(a, SL, k, s);
     return hipGetLastError() == hipSuccess ? MF_SUCCESS : MF_ERR_HIP;
 }
 

@@ -120,9 +120,11 @@ mf_status row_streams(mf_matrix *A, bool mixed, hipStream_t s, RowStreams *out)
         }
         it = L.parts.emplace(-rpt, P).first;
     }
-    mf_status st = ensure_sell(A, &it->second, rpt, mixed, s, &out->S, &out->narrow, false);
+    const SellLayout *SL = nullptr;
+    mf_status st = ensure_sell(A, &it->second, rpt, mixed, s, &out->S, &SL, false);
     if (st == MF_SUCCESS) st = L.ensure_tile_order(s);
     if (st != MF_SUCCESS) return st;
+    out->narrow = SL->narrow;
     out->L = &L;
     out->P = &it->second;
     out->rpt = rpt;

@@ -460,14 +460,15 @@ mf_status bicg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_sol
     if ((st = A->ws.ensure(std::max(A->L.n_rows, A->L.n_cols), G, s)) != MF_SUCCESS) return st;
     mfk::DevSell dsell;
     memset(&dsell, 0, sizeof(dsell));
-    bool narrow = false;
-    if (sell && (st = ensure_sell(A, P, rpt, mixed, s, &dsell, &narrow, rpt >= 4)) != MF_SUCCESS) return st;
+    const SellLayout *SL = nullptr;
+    if (sell && (st = ensure_sell(A, P, rpt, mixed, s, &dsell, &SL, rpt >= 4)) != MF_SUCCESS) return st;
+    const bool narrow = SL && SL->narrow;
     // as in the CG launcher: binary64 arithmetic when the class streams would not move fewer
     // bytes than the binary64 stream
     bool mixed_arith = mixed;
     if (sell && mixed && o->layout == 0) {
         double bc = 0, b64 = 0;
-        sell_bytes(P, &bc, &b64);
+        sell_bytes(*SL, &bc, &b64);
         if (bc >= 0.95 * b64) mixed_arith = false;
     }
     BicgKernel k = nullptr;
@@ -481,7 +482,7 @@ mf_status bicg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_sol
     bool on_chip = false;
     if (k && sell && !mixed_arith && !dsell.perm && o->value_cache == 0) {
         size_t offs[mfk::kSellStreams];
-        const size_t need = sell_lds_bytes(*P->sell, false, offs, lds);
+        const size_t need = sell_lds_bytes(*SL, false, offs, lds);
         BicgKernel kl = pick_bicg<0, 1 | mfk::kSellLds64>(rpt);
         // (4 KB left for the kernel's static LDS)
         if (kl && need + 4096 <= (size_t)A->max_lds) {

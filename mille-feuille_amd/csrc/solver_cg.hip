@@ -297,7 +297,7 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     if (ext && var == 3) return MF_ERR_UNSUPPORTED;  // no second publish buffer pair in the scratch
     mfk::DevSell dsell;
     memset(&dsell, 0, sizeof(dsell));
-    bool narrow = false;
+    const SellLayout *SL = nullptr;
     const bool perm_ok = cg_perm_supported(rpt, var) && A->L.n_rows > kPermMinRows * G;
     // A tile-mixed solve whose binary64 stream fits the workgroups' LDS runs binary64
     // arithmetic on it (reported in info->precision): with the values on chip the SpMV waits
@@ -307,19 +307,20 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     // 7.1 / 6.9.  The arithmetic does not depend on value_cache, so both settings agree.
     bool mixed_arith = mixed;
     if (sell && mixed && var == 4 && o->layout == 0 && small64) {
-        if ((st = ensure_sell(A, P, rpt, false, s, &dsell, &narrow, perm_ok, !ext)) != MF_SUCCESS) return st;
+        if ((st = ensure_sell(A, P, rpt, false, s, &dsell, &SL, perm_ok, !ext)) != MF_SUCCESS) return st;
         size_t offs[mfk::kSellStreams];
-        if (!dsell.perm && cg_sell_lds_kernel_for(rpt, false, narrow) &&
-            sell_lds_bytes(*P->sell, false, offs, lds_x) + 4096 <= (size_t)A->max_lds)
+        if (!dsell.perm && cg_sell_lds_kernel_for(rpt, false, SL->narrow) &&
+            sell_lds_bytes(*SL, false, offs, lds_x) + 4096 <= (size_t)A->max_lds)
             mixed_arith = false;
     }
-    if (sell && (st = ensure_sell(A, P, rpt, mixed_arith, s, &dsell, &narrow, perm_ok, !ext)) != MF_SUCCESS) return st;
+    if (sell && (st = ensure_sell(A, P, rpt, mixed_arith, s, &dsell, &SL, perm_ok, !ext)) != MF_SUCCESS) return st;
+    const bool narrow = SL && SL->narrow;
     // Tile-mixed solve whose class streams would move about as many bytes as the binary64
     // stream (rows spread over classes pad each class stream): binary64 arithmetic on the
     // binary64 stream is then as fast and exact; reported in info->precision.
     if (sell && mixed_arith && o->layout == 0) {
         double bc = 0, b64 = 0;
-        sell_bytes(P, &bc, &b64);
+        sell_bytes(*SL, &bc, &b64);
         if (bc >= 0.95 * b64) mixed_arith = false;
     }
     CgKernel k = sell ? cg_sell_kernel_for(rpt, var, mixed_arith, narrow, dsell.perm != nullptr) : nullptr;
@@ -330,7 +331,7 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     bool on_chip = false;
     if (sell && k && var == 4 && !dsell.perm && o->value_cache == 0) {
         size_t offs[mfk::kSellStreams];
-        const size_t need = sell_lds_bytes(*P->sell, mixed_arith, offs, lds_x);
+        const size_t need = sell_lds_bytes(*SL, mixed_arith, offs, lds_x);
         CgKernel kl = cg_sell_lds_kernel_for(rpt, mixed_arith, narrow);
         // (4 KB left for the kernel's static LDS: reduction partials and flags)
         if (kl && need + 4096 <= (size_t)A->max_lds) {
@@ -351,28 +352,27 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     // workgroup always takes the window: p then never leaves the CU.
     bool window = false;
     if (sell && k && var == 4) {
-        const SellLayout &SL = *P->sell;
         int64_t units = 0, shared = 0;
         for (int s2 = 0; s2 < mfk::kSellStreams; s2++)
             if (mixed_arith == (s2 != mfk::kSellAll64)) {
-                units += SL.units[s2];
-                shared += SL.shared_units[s2];
+                units += SL->units[s2];
+                shared += SL->shared_units[s2];
             }
         const size_t at = (lds + 15) / 16 * 16;
-        const size_t need = at + (size_t)SL.max_win[mixed_arith] * (mixed_arith ? 4 : 8);
+        const size_t need = at + (size_t)SL->max_win[mixed_arith] * (mixed_arith ? 4 : 8);
         CgKernel kw = cg_sell_win_kernel_for(rpt, mixed_arith, narrow, dsell.perm != nullptr, on_chip);
-        const bool reuse = 2 * shared < units && (int64_t)SL.max_win[mixed_arith] <= 4 * (A->L.nnz / G);
+        const bool reuse = 2 * shared < units && (int64_t)SL->max_win[mixed_arith] <= 4 * (A->L.nnz / G);
         if (kw && (G == 1 || reuse) && need + 4096 <= (size_t)A->max_lds) {
             k = kw;
             lds = need;
-            dsell.win = SL.win[mixed_arith];
+            dsell.win = SL->win[mixed_arith];
             dsell.win_lds = (int)at;
             window = true;
         }
     }
     if (sell && ((!k && dsell.perm) || (fp64_small && var == 4 && !on_chip))) {
-        // the partition's streams were built permuted for another variant, or an all-FP64
-        // stream chosen for LDS residency did not fit: tile chunks
+        // streams of sorted rows and no kernel for them, or an all-FP64 stream chosen for LDS
+        // residency did not fit: tile chunks
         on_chip = window = false;
         sell = false;
         mixed_arith = mixed;

@@ -24,7 +24,6 @@ struct SellLayout {
     bool mixed = false;             // streams 0..3 built (stream 4 always)
     bool narrow = false;            // unit profile of streams 1..3 (sell.h)
     bool permuted = false;          // rows sorted by length within each range
-    bool ordered = false;           // the row order of this partition has been decided
     std::vector<int> h_perm;        // host: local row of each thread slot, per range (permuted)
     int *perm = nullptr;            // device copy when permuted
     int64_t units[mfk::kSellStreams] = {0, 0, 0, 0, 0};
@@ -51,7 +50,11 @@ struct Partition {
     long long *wg_chunk = nullptr;  // device, 4G+1
     int3 *chunks = nullptr;         // device, class-sorted headers
     std::vector<int> h_tr;          // host copy of wg_tr
-    SellLayout *sell = nullptr;     // built on first use by a sliced-ELL solve
+    // streams built on first use by a sliced-ELL solve: [0] rows in order, [1] each range's
+    // rows sorted by length (for the launchers that have kernels for them, when sorting pays:
+    // -1 not looked at yet, 0 no, 1 yes).  Two caches: one solver's order is not another's
+    SellLayout *sell[2] = {nullptr, nullptr};
+    int sort_pays = -1;
     // ranges owning the columns of each range's entries (itself excluded):
     // dep_idx[dep_ptr[r] .. dep_ptr[r+1]), device
     int *dep_ptr = nullptr, *dep_idx = nullptr;
@@ -109,13 +112,14 @@ struct DeviceLayout {
 // of the range, the rows being permuted).
 bool sell_supported(const mf_matrix *A, int rpt);
 // Sliced-ELL streams of partition P for rpt rows per thread (built and cached on first
-// use; `mixed` also builds the per-class streams); *narrow receives their unit profile and
-// out->perm the row permutation (null: identity), which the first build may choose only
-// when allow_perm (the caller has kernels for it).
+// use; `mixed` also builds the per-class streams); *layout receives the streams used and
+// out->perm their row permutation (null: identity), which needs allow_perm (the caller has
+// kernels for it) and sorting to pay.  At 4 or more rows per thread a caller without allow_perm
+// may get the permutation of streams that are there, and has to take the tile chunks then.
 // With build = false nothing is built or freed: MF_ERR_UNSUPPORTED when the streams an
 // earlier call built do not cover (rpt, mixed).
 mf_status ensure_sell(mf_matrix *A, const Partition *P, int rpt, bool mixed, hipStream_t s, mfk::DevSell *out,
-                      bool *narrow, bool allow_perm, bool build = true);
+                      const SellLayout **layout, bool allow_perm, bool build = true);
 // The streams of `mask` built on the GPU, for ranges that keep their row order
 // (sell_build.hip).
 mf_status build_sell_gpu(mf_matrix *A, const Partition &P, SellLayout &SL, unsigned mask, hipStream_t s);
@@ -123,8 +127,8 @@ mf_status build_sell_gpu(mf_matrix *A, const Partition &P, SellLayout &SL, unsig
 // (built on the host) are dropped instead, and rebuilt by the next solve that uses them.
 mf_status refill_sell(mf_matrix *A, Partition &P, hipStream_t s);
 // Padded bytes of one pass over the built class streams (0..3) and over the binary64
-// stream (4) of P's sliced-ELL layout.
-void sell_bytes(const Partition *P, double *class_streams, double *all64);
+// stream (4) of a sliced-ELL layout.
+void sell_bytes(const SellLayout &SL, double *class_streams, double *all64);
 size_t sell_lds_bytes(const SellLayout &SL, bool mixed_arith, size_t offsets[mfk::kSellStreams], size_t base);
 
 
