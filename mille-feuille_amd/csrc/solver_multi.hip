@@ -334,8 +334,10 @@ mf_status mk_setup(mf_matrix *A, const mf_solve_options *o, hipStream_t s, MkCtx
     c.n = A->L.n_rows;
     c.mixed = o->precision == MF_PREC_MIXED && A->L.has_lowp;
     if (A->L.tilem == 0 || A->L.n_rows != A->L.n_cols) return MF_ERR_INVALID;
-    mf_status rst = row_streams(A, c.mixed, s, &c.rows);
-    if (rst != MF_SUCCESS) return rst;
+    if (o->layout != 1) {  // 1: the caller asked for the tile chunks
+        const mf_status rst = row_streams(A, c.mixed, s, &c.rows);
+        if (rst != MF_SUCCESS) return rst;
+    }
     c.partial = c.alloc<double>(mfk::kDotBlocks);
     c.sc = c.alloc<double>(32);
     if (!c.partial || !c.sc) return MF_ERR_ALLOC;
