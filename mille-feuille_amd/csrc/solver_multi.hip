@@ -29,12 +29,19 @@ namespace mfk {
 
 constexpr int kDotBlocks = 512;
 
+// State of a multi-kernel CG, in the solve's 32 scalars.
+enum { MKS_RR = 0, MKS_IT = 1, MKS_STATE = 2 };
+enum { MK_RUN = 0, MK_CHECK = 1, MK_BREAK = 2, MK_MAXIT = 3 };
+
 // PM: product mode of the tile-mixed SpMV (sell.h): kPmLow32 for CG, kPmWide64 for
-// BiCGSTAB, as in the persistent kernels.
+// BiCGSTAB, as in the persistent kernels.  sc: the state of the CG whose batch of iterations
+// the product belongs to (nothing is done once it is decided), or null.
 template <bool MIXED, int PM>
 __global__ __launch_bounds__(1024) void mk_spmv(DevMatrix A, const double *__restrict__ x64,
-                                                const float *__restrict__ x32, double *__restrict__ y)
+                                                const float *__restrict__ x32, double *__restrict__ y,
+                                                const double *sc)
 {
+    if (sc && sc[MKS_STATE] != (double)MK_RUN) return;
     extern __shared__ double q[];
     __shared__ double qdummy[64];
     const int w = blockIdx.x;
@@ -71,9 +78,6 @@ __global__ __launch_bounds__(256) void mk_finish(const double *__restrict__ part
     if (threadIdx.x == 0) *out = s[0] + s[1] + s[2] + s[3];
 }
 
-// State of a multi-kernel CG, in the solve's 32 scalars.
-enum { MKS_RR = 0, MKS_IT = 1, MKS_STATE = 2 };
-enum { MK_RUN = 0, MK_CHECK = 1, MK_BREAK = 2, MK_MAXIT = 3 };
 constexpr int kUpdBlocks = 512, kUpdThreads = 512;
 
 // q = A p over row streams, range blockIdx.x, + gridDim.x, ...; part[4 b ..] = this
@@ -300,17 +304,19 @@ struct MkCtx {
         bufs.push_back(p);
         return (T *)p;
     }
-    // use_mixed: tile classes with product mode pm (kPmLow32 CG, kPmWide64 BiCGSTAB)
-    void spmv(const double *x64, const float *x32, double *y, bool use_mixed, int pm = mfk::kPmLow32)
+    // use_mixed: tile classes with product mode pm (kPmLow32 CG, kPmWide64 BiCGSTAB); state:
+    // mk_spmv's sc
+    void spmv(const double *x64, const float *x32, double *y, bool use_mixed, int pm = mfk::kPmLow32,
+              const double *state = nullptr)
     {
         if (rows.ok)
             row_spmv(rows, n, x64, x32, y, use_mixed, pm, s);
         else if (use_mixed && pm == mfk::kPmWide64)
-            hipLaunchKernelGGL((mfk::mk_spmv<true, mfk::kPmWide64>), dim3(G), dim3(1024), lds, s, dm, x64, x32, y);
+            hipLaunchKernelGGL((mfk::mk_spmv<true, mfk::kPmWide64>), dim3(G), dim3(1024), lds, s, dm, x64, x32, y, state);
         else if (use_mixed)
-            hipLaunchKernelGGL((mfk::mk_spmv<true, mfk::kPmLow32>), dim3(G), dim3(1024), lds, s, dm, x64, x32, y);
+            hipLaunchKernelGGL((mfk::mk_spmv<true, mfk::kPmLow32>), dim3(G), dim3(1024), lds, s, dm, x64, x32, y, state);
         else
-            hipLaunchKernelGGL((mfk::mk_spmv<false, mfk::kPmTiles>), dim3(G), dim3(1024), lds, s, dm, x64, x32, y);
+            hipLaunchKernelGGL((mfk::mk_spmv<false, mfk::kPmTiles>), dim3(G), dim3(1024), lds, s, dm, x64, x32, y, state);
     }
     void dot(const double *a, const double *b, int slot)
     {
@@ -388,7 +394,7 @@ void fill_info(mf_solve_info *info, const MkCtx &c, int status, int it, int repl
 static int mk_cg_product(MkCtx &c, const double *p, const float *p32, const double *r, double *q, double *part)
 {
     if (!c.rows.ok) {
-        c.spmv(p, p32, q, c.mixed);
+        c.spmv(p, p32, q, c.mixed, mfk::kPmLow32, c.sc);
         hipLaunchKernelGGL(mfk::mk_cg_dots, dim3(mfk::kDotBlocks), dim3(1024), 0, c.s, c.n, p, r, q, part, c.sc);
         return mfk::kDotBlocks;
     }
@@ -442,29 +448,35 @@ mf_status cg_multikernel(mf_matrix *A, const double *b, double *x, const mf_solv
     const int max_repl = o->max_replacements > 0 ? o->max_replacements : 64;
     if (bb == 0.0) status = MF_SUCCESS;
     constexpr int kBatch = 16;
+    bool rr_of_r = true;  // rr is r'r of the present r (at the start, after a replacement)
     while (status == MF_NOT_CONVERGED) {
         // r'r at or below which the host decides; a tile-mixed solve also looks before the
         // strict bound dl^2 rbase of a replacement, and at exactly that value goes on
         const bool may_replace = c.mixed && repl < max_repl;
         const double below = std::nextafter(dl * dl * rbase, 0.0);
         const double check2 = o->fixed_iterations ? -1.0 : may_replace ? std::max(tol2 * bb, below) : tol2 * bb;
-        int last = it;
-        for (int i = 0; i < kBatch && last <= o->max_iter; i++, last++) {
-            const int parts = mk_cg_product(c, p, p32, r, q, part);
-            hipLaunchKernelGGL(mfk::mk_cg_update, dim3(mfk::kUpdBlocks), dim3(mfk::kUpdThreads), 0, s, n, parts, part,
-                               check2, last, o->max_iter, x, r, p, p32, q, c.sc);
-        }
-        double h[3];
-        if (hipMemcpyAsync(h, c.sc, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            return MF_ERR_HIP;
-        rr = h[mfk::MKS_RR];
-        const int state = (int)h[mfk::MKS_STATE];
+        int state = mfk::MK_RUN;
+        if (rr_of_r) state = rr <= check2 ? mfk::MK_CHECK : it >= o->max_iter ? mfk::MK_MAXIT : mfk::MK_RUN;
         if (state == mfk::MK_RUN) {
-            it = last;
-            continue;
+            int last = it;
+            for (int i = 0; i < kBatch && last <= o->max_iter; i++, last++) {
+                const int parts = mk_cg_product(c, p, p32, r, q, part);
+                hipLaunchKernelGGL(mfk::mk_cg_update, dim3(mfk::kUpdBlocks), dim3(mfk::kUpdThreads), 0, s, n, parts,
+                                   part, check2, last, o->max_iter, x, r, p, p32, q, c.sc);
+            }
+            double h[3];
+            if (hipMemcpyAsync(h, c.sc, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
+                hipStreamSynchronize(s) != hipSuccess)
+                return MF_ERR_HIP;
+            rr = h[mfk::MKS_RR];
+            rr_of_r = false;
+            state = (int)h[mfk::MKS_STATE];
+            if (state == mfk::MK_RUN) {
+                it = last;
+                continue;
+            }
+            it = (int)h[mfk::MKS_IT];
         }
-        it = (int)h[mfk::MKS_IT];
         if (state == mfk::MK_BREAK) {
             status = MF_BREAKDOWN;
         } else if (state == mfk::MK_MAXIT) {
@@ -478,6 +490,7 @@ mf_status cg_multikernel(mf_matrix *A, const double *b, double *x, const mf_solv
             hipLaunchKernelGGL(mfk::mk_residual, vg, dim3(256), 0, s, b, q, r, p, p32, n);
             c.dot(r, r, 4);
             rr = rbase = c.read(4);
+            rr_of_r = true;
             repl++;
             if (rr <= tol2 * bb) status = MF_SUCCESS;
             else if (hipMemsetAsync(c.sc + mfk::MKS_STATE, 0, sizeof(double), s) != hipSuccess) return MF_ERR_HIP;
