@@ -92,6 +92,15 @@ static double rows_padding(const mf_matrix *A)
 // Most padding with which the row streams still beat the tile chunks.
 constexpr double kRowsPadding = 1.6;
 
+// Streams that do not fit the device memory: the tile chunks, which are there already, from
+// now on (a matrix created or given new values on the host tries the streams again).
+static mf_status no_streams(DeviceLayout &L)
+{
+    (void)hipGetLastError();  // the refused allocation is not the next launch's error
+    L.rows_regular = 0;
+    return MF_SUCCESS;
+}
+
 mf_status row_streams(mf_matrix *A, bool mixed, hipStream_t s, RowStreams *out)
 {
     out->ok = false;
@@ -116,13 +125,14 @@ mf_status row_streams(mf_matrix *A, bool mixed, hipStream_t s, RowStreams *out)
         const mf_status st = upload((void **)&P.wg_tr, P.h_tr.data(), sizeof(int) * P.h_tr.size(), s);
         if (st != MF_SUCCESS || hipStreamSynchronize(s) != hipSuccess) {
             free_partition(P);
-            return st != MF_SUCCESS ? st : MF_ERR_HIP;
+            return st == MF_ERR_ALLOC ? no_streams(L) : st != MF_SUCCESS ? st : MF_ERR_HIP;
         }
         it = L.parts.emplace(-rpt, P).first;
     }
     const SellLayout *SL = nullptr;
     mf_status st = ensure_sell(A, &it->second, rpt, mixed, s, &out->S, &SL, false);
     if (st == MF_SUCCESS) st = L.ensure_tile_order(s);
+    if (st == MF_ERR_ALLOC || st == MF_ERR_TOO_LARGE) return no_streams(L);
     if (st != MF_SUCCESS) return st;
     out->narrow = SL->narrow;
     out->L = &L;
