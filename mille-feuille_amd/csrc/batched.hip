@@ -578,7 +578,7 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
     const SellLayout *layout = nullptr;
     if (o.layout != 1 && sell_supported(A, rpt)) {
         bool taken = false;
-        if (ensure_sell(A, &B->part, rpt, mixed, s, &dsell, &layout, false, true) == MF_SUCCESS) {
+        if (ensure_sell(A, &B->part, rpt, sell_need(mixed), s, &dsell, &layout, false, true) == MF_SUCCESS) {
             auto take = [&](BatchKernel ks, size_t bytes) {
                 int occ2 = 0;
                 if (!ks ||

@@ -700,7 +700,7 @@ size_t sell_lds_bytes(const SellLayout &SL, bool mixed_arith, size_t offsets[mfk
     return off;
 }
 
-mf_status ensure_sell(mf_matrix *A, const Partition *Pc, int rpt, bool mixed, hipStream_t s, mfk::DevSell *out,
+mf_status ensure_sell(mf_matrix *A, const Partition *Pc, int rpt, unsigned need, hipStream_t s, mfk::DevSell *out,
                       const SellLayout **layout, bool allow_perm, bool build)
 {
     // the sliced-ELL streams are a cache of the partition, rebuilt with it
@@ -720,7 +720,8 @@ mf_status ensure_sell(mf_matrix *A, const Partition *Pc, int rpt, bool mixed, hi
         return MF_SUCCESS;
     }
     SellLayout *&cache = P.sell[allow_perm && P.sort_pays == 1 ? 1 : 0];
-    if (!build && (!cache || cache->rpt != rpt || !cache->soff[mfk::kSellAll64] || (mixed && !cache->mixed)))
+    if (!build && (!cache || cache->rpt != rpt || ((need & kNeed64) && !cache->soff[mfk::kSellAll64]) ||
+                   ((need & kNeedClasses) && !cache->mixed)))
         return MF_ERR_UNSUPPORTED;
     if (!cache) {
         cache = new SellLayout();
@@ -728,8 +729,8 @@ mf_status ensure_sell(mf_matrix *A, const Partition *Pc, int rpt, bool mixed, hi
     }
     SellLayout &SL = *cache;
     unsigned mask = 0;
-    if (!SL.soff[mfk::kSellAll64]) mask |= 1u << mfk::kSellAll64;
-    if (mixed && !SL.mixed) mask |= 0xFu;
+    if ((need & kNeed64) && !SL.soff[mfk::kSellAll64]) mask |= 1u << mfk::kSellAll64;
+    if ((need & kNeedClasses) && !SL.mixed) mask |= 0xFu;
     if (mask) {
         mf_status st = SL.permuted ? host_values(A, s) : MF_SUCCESS;
         if (st == MF_SUCCESS) st = SL.permuted ? build_sell(A, P, SL, mask, s) : build_sell_gpu(A, P, SL, mask, s);
@@ -1061,7 +1062,7 @@ extern "C" mf_status mf_spmv(mf_matrix *A, const double *d_x, double *d_y, int p
     // (the tile-chunk path's bound: a range's rows on num_cus workgroups fit their LDS)
     if ((int64_t)A->L.n_rows * 8 > (int64_t)A->max_lds * A->num_cus) return MF_ERR_TOO_LARGE;
     RowStreams R;
-    mf_status st = row_streams(A, mixed, s, &R);
+    mf_status st = row_streams(A, mixed ? kNeedClasses : kNeed64, s, &R);
     if (st != MF_SUCCESS) return st;
     if (R.ok) {
         if (mixed) {

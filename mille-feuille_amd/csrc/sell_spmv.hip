@@ -101,7 +101,7 @@ static mf_status no_streams(DeviceLayout &L)
     return MF_SUCCESS;
 }
 
-mf_status row_streams(mf_matrix *A, bool mixed, hipStream_t s, RowStreams *out)
+mf_status row_streams(mf_matrix *A, unsigned need, hipStream_t s, RowStreams *out)
 {
     out->ok = false;
     DeviceLayout &L = A->L;
@@ -109,7 +109,7 @@ mf_status row_streams(mf_matrix *A, bool mixed, hipStream_t s, RowStreams *out)
     // Rows per thread.  Binary64 rows fill the pipeline with one slice a wave, and more waves
     // hide more (3D 127 x 129 x 125: 35.8 / 37.8 / 43.9 us at 1 / 2 / 4 rows); of the class
     // streams a slice is a unit or two, so large matrices take four (35.5 / 27.9 / 27.8 us).
-    int rpt = mixed && L.n_rows >= (1 << 19) ? 4 : 1;
+    int rpt = (need & kNeedClasses) && L.n_rows >= (1 << 19) ? 4 : 1;
     while (rpt > 1 && !sell_supported(A, rpt)) rpt /= 2;
     if (!sell_supported(A, rpt)) return MF_SUCCESS;
     if (L.rows_regular < 0) L.rows_regular = rows_padding(A) <= kRowsPadding;
@@ -130,7 +130,7 @@ mf_status row_streams(mf_matrix *A, bool mixed, hipStream_t s, RowStreams *out)
         it = L.parts.emplace(-rpt, P).first;
     }
     const SellLayout *SL = nullptr;
-    mf_status st = ensure_sell(A, &it->second, rpt, mixed, s, &out->S, &SL, false);
+    mf_status st = ensure_sell(A, &it->second, rpt, need, s, &out->S, &SL, false);
     if (st == MF_SUCCESS) st = L.ensure_tile_order(s);
     if (st == MF_ERR_ALLOC || st == MF_ERR_TOO_LARGE) return no_streams(L);
     if (st != MF_SUCCESS) return st;

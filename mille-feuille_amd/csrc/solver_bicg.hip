@@ -461,7 +461,7 @@ mf_status bicg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_sol
     mfk::DevSell dsell;
     memset(&dsell, 0, sizeof(dsell));
     const SellLayout *SL = nullptr;
-    if (sell && (st = ensure_sell(A, P, rpt, mixed, s, &dsell, &SL, rpt >= 4)) != MF_SUCCESS) return st;
+    if (sell && (st = ensure_sell(A, P, rpt, sell_need(mixed), s, &dsell, &SL, rpt >= 4)) != MF_SUCCESS) return st;
     const bool narrow = SL && SL->narrow;
     // as in the CG launcher: binary64 arithmetic when the class streams would not move fewer
     // bytes than the binary64 stream

@@ -307,13 +307,13 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     // 7.1 / 6.9.  The arithmetic does not depend on value_cache, so both settings agree.
     bool mixed_arith = mixed;
     if (sell && mixed && var == 4 && o->layout == 0 && small64) {
-        if ((st = ensure_sell(A, P, rpt, false, s, &dsell, &SL, perm_ok, !ext)) != MF_SUCCESS) return st;
+        if ((st = ensure_sell(A, P, rpt, kNeed64, s, &dsell, &SL, perm_ok, !ext)) != MF_SUCCESS) return st;
         size_t offs[mfk::kSellStreams];
         if (!dsell.perm && cg_sell_lds_kernel_for(rpt, false, SL->narrow) &&
             sell_lds_bytes(*SL, false, offs, lds_x) + 4096 <= (size_t)A->max_lds)
             mixed_arith = false;
     }
-    if (sell && (st = ensure_sell(A, P, rpt, mixed_arith, s, &dsell, &SL, perm_ok, !ext)) != MF_SUCCESS) return st;
+    if (sell && (st = ensure_sell(A, P, rpt, sell_need(mixed_arith), s, &dsell, &SL, perm_ok, !ext)) != MF_SUCCESS) return st;
     const bool narrow = SL && SL->narrow;
     // Tile-mixed solve whose class streams would move about as many bytes as the binary64
     // stream (rows spread over classes pad each class stream): binary64 arithmetic on the

@@ -21,7 +21,7 @@ namespace mf {
 // units[s] units; soff[s] holds the first unit of every (range, wave, slice) slot.
 struct SellLayout {
     int rpt = 0;
-    bool mixed = false;             // streams 0..3 built (stream 4 always)
+    bool mixed = false;             // streams 0..3 built (stream 4: soff not null)
     bool narrow = false;            // unit profile of streams 1..3 (sell.h)
     bool permuted = false;          // rows sorted by length within each range
     std::vector<int> h_perm;        // host: local row of each thread slot, per range (permuted)
@@ -111,14 +111,18 @@ struct DeviceLayout {
 // streams: every column within the 16-bit offset range of its lane's slot-0 row (any row
 // of the range, the rows being permuted).
 bool sell_supported(const mf_matrix *A, int rpt);
-// Sliced-ELL streams of partition P for rpt rows per thread (built and cached on first
-// use; `mixed` also builds the per-class streams); *layout receives the streams used and
+// Which streams a call reads: the binary64 stream, the class streams (tile-mixed products), or
+// both (tile-mixed solves, whose residuals are binary64).
+enum { kNeed64 = 1, kNeedClasses = 2 };
+inline unsigned sell_need(bool mixed) { return mixed ? kNeed64 | kNeedClasses : kNeed64; }
+// Sliced-ELL streams of partition P for rpt rows per thread (those of `need`, built and cached
+// on first use); *layout receives the streams used and
 // out->perm their row permutation (null: identity), which needs allow_perm (the caller has
 // kernels for it) and sorting to pay.  At 4 or more rows per thread a caller without allow_perm
 // may get the permutation of streams that are there, and has to take the tile chunks then.
 // With build = false nothing is built or freed: MF_ERR_UNSUPPORTED when the streams an
-// earlier call built do not cover (rpt, mixed).
-mf_status ensure_sell(mf_matrix *A, const Partition *P, int rpt, bool mixed, hipStream_t s, mfk::DevSell *out,
+// earlier call built do not cover (rpt, need).
+mf_status ensure_sell(mf_matrix *A, const Partition *P, int rpt, unsigned need, hipStream_t s, mfk::DevSell *out,
                       const SellLayout **layout, bool allow_perm, bool build = true);
 // The streams of `mask` built on the GPU, for ranges that keep their row order
 // (sell_build.hip).
@@ -134,7 +138,8 @@ size_t sell_lds_bytes(const SellLayout &SL, bool mixed_arith, size_t offsets[mfk
 
 // Sliced-ELL streams over ranges of 1024 rpt consecutive rows for products launched by
 // themselves (sell_spmv.hip), built on first use; ok = false: the matrix keeps the tile chunks
-// (not square, columns beyond the 16-bit offsets, or rows of very different lengths).
+// (not square, columns beyond the 16-bit offsets, rows of very different lengths, or no device
+// memory for the streams).
 struct RowStreams {
     bool ok = false;
     const DeviceLayout *L = nullptr;
@@ -143,7 +148,7 @@ struct RowStreams {
     bool narrow = false;
     int rpt = 0;
 };
-mf_status row_streams(mf_matrix *A, bool mixed, hipStream_t s, RowStreams *out);
+mf_status row_streams(mf_matrix *A, unsigned need, hipStream_t s, RowStreams *out);
 // y = A x: binary64 values and x64, or (mixed) the tile classes under product mode pm.
 void row_spmv(const RowStreams &R, int n, const double *x64, const float *x32, double *y, bool mixed, int pm,
               hipStream_t s);

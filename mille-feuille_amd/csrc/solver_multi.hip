@@ -341,7 +341,7 @@ mf_status mk_setup(mf_matrix *A, const mf_solve_options *o, hipStream_t s, MkCtx
     c.mixed = o->precision == MF_PREC_MIXED && A->L.has_lowp;
     if (A->L.tilem == 0 || A->L.n_rows != A->L.n_cols) return MF_ERR_INVALID;
     if (o->layout != 1) {  // 1: the caller asked for the tile chunks
-        const mf_status rst = row_streams(A, c.mixed, s, &c.rows);
+        const mf_status rst = row_streams(A, sell_need(c.mixed), s, &c.rows);
         if (rst != MF_SUCCESS) return rst;
     }
     c.partial = c.alloc<double>(mfk::kDotBlocks);

@@ -88,3 +88,26 @@ def test_tile_chunks_when_streams_do_not_fit(mf, torch, tmp_path):
     r = subprocess.run([sys.executable, str(tmp_path / "child.py"), str(tmp_path / "shim.so"), str(root), str(root / "oracle")],
                        capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "mixed ok" in r.stdout, r.stdout + r.stderr
+
+
+def test_tile_mixed_product_builds_no_binary64_stream(mf, torch):
+    """Device memory of the first tile-mixed product: the class streams and the workspace, not
+    the binary64 stream that it does not read (80 bytes a row here)."""
+    rp, ci, va = mf.workloads.poisson3d(100)
+    n = rp.size - 1
+    A = mf.TiledMatrix(rp, ci, va)
+    x = torch.rand(n, dtype=torch.float64, device="cuda")
+    y = torch.empty_like(x)
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    A.spmv(x, precision="mixed", out=y)
+    torch.cuda.synchronize()
+    used = before - torch.cuda.mem_get_info()[0]
+    print(f"{used / n:.1f} bytes a row", flush=True)
+    assert used < 110 * n
+    # the other streams follow when they are asked for
+    z = A.spmv(x)
+    assert torch.allclose(y, z, rtol=0, atol=12 * 2.0 ** -23)
+    xs, info = A.cg_multikernel(z, tol=1e-10, precision="mixed")
+    assert info["status"] == 0 and info["precision"] == 1 and info["layout"] in (2, 3)
+    A.close()
