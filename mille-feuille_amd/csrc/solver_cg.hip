@@ -234,6 +234,14 @@ int default_grid(const mf_matrix *A, int maxG, int cg_rows)
     return (int)g;
 }
 
+// Whether an earlier call built sliced-ELL streams over one workgroup (a solve without
+// allocation takes the plan that exists).
+static bool one_group_plan(const mf_matrix *A)
+{
+    const Partition *P = A->L.find_partition(1);
+    return P && (P->sell[0] || P->sell[1]);
+}
+
 // ext: run on these buffers instead of the matrix's workspace, building nothing (the
 // partition and SpMV streams must exist from an earlier solve) and allocating nothing
 // (no workspace growth, no timing events: info->time_ms is 0).
@@ -249,7 +257,7 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     if (A->L.tilem == 0) return MF_ERR_INVALID;
     // (pipelined CG holds five row vectors: at most 2 rows per thread, so the chunk rule)
     const long long tuned = ((long long)(req ? req : 2) << 8) | (mixed ? 1 : 0);
-    const bool tiny = tiny_ok && o->grid == 0 && A->tuned_grid.find(tuned) == A->tuned_grid.end() &&
+    const bool tiny = tiny_ok && (!ext || one_group_plan(A)) && o->grid == 0 && A->tuned_grid.find(tuned) == A->tuned_grid.end() &&
                       (o->variant == 0 || o->variant == 4) && !dyn && o->layout != 1 && o->value_cache == 0 &&
                       A->L.n_rows <= kTinyRows && A->L.nnz <= kTinyNnz;
     const int G = tiny ? 1 : choose_grid(A, o, tuned, dyn || req == 3 ? 0 : 1024);
