@@ -121,10 +121,11 @@ static CgKernel pick_cg_perm(int rpt)
     }
 }
 
-// Sorting needs slices to sort into: ranges of about two slices only pay for the indirection (graph
-// Laplacian, us per iteration sorted / in order: 78 rows a range 12.9 / 12.4, 234 rows
-// 15.8 / 20.6, 1,172 rows 41 / 53).
-constexpr int kPermMinRows = 128;
+// Rows a range must hold on average for its rows to be sorted and p to be gathered from an LDS
+// window.  Sorting needs slices to sort into: ranges of about two slices only pay for the
+// indirection (graph Laplacian, us per iteration sorted / in order: 78 rows a range 12.9 / 12.4,
+// 234 rows 15.8 / 20.6, 1,172 rows 41 / 53).
+constexpr int kRangeMinRows = 128;
 
 static bool cg_perm_supported(int rpt, int var) { return (var == 2 || var == 4) && rpt <= 8; }
 
@@ -306,7 +307,7 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     mfk::DevSell dsell;
     memset(&dsell, 0, sizeof(dsell));
     const SellLayout *SL = nullptr;
-    const bool perm_ok = cg_perm_supported(rpt, var) && A->L.n_rows > kPermMinRows * G;
+    const bool perm_ok = cg_perm_supported(rpt, var) && A->L.n_rows > kRangeMinRows * G;
     // A tile-mixed solve whose binary64 stream fits the workgroups' LDS runs binary64
     // arithmetic on it (reported in info->precision): with the values on chip the SpMV waits
     // for units, not bytes, class streams start their pipelines one after another, and no
@@ -355,7 +356,10 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     // bounds the SpMV; the window is read in whole lines, once, and the gathers go to LDS
     // (graph Laplacian of 300,007 rows, 21 entries a row within 8,000: 41 -> 26 us per
     // iteration).  Where the workgroup's entries are few next to its window, loading it costs
-    // more than it saves: 3.5 columns an entry 14.3 -> 13.1 us, 12 an entry 12.3 -> 13.7.
+    // more than it saves: 3.5 columns an entry 14.3 -> 13.1 us, 12 an entry 12.3 -> 13.7; and so
+    // it does in ranges of a slice or two, however narrow (78 rows a range, 21 entries a row:
+    // 200 columns either side 11.8 -> 12.2, 2,000 either side 15.0 -> 15.8 in binary64 and
+    // 16.1 -> 16.9 on class streams in LDS).
     // Stencil waves (shared column offsets) gather whole lines as it is.  A grid of one
     // workgroup always takes the window: p then never leaves the CU.
     bool window = false;
@@ -369,7 +373,7 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
         const size_t at = (lds + 15) / 16 * 16;
         const size_t need = at + (size_t)SL->max_win[mixed_arith] * (mixed_arith ? 4 : 8);
         CgKernel kw = cg_sell_win_kernel_for(rpt, mixed_arith, narrow, dsell.perm != nullptr, on_chip);
-        const bool reuse = 2 * shared < units && (int64_t)SL->max_win[mixed_arith] <= 4 * (A->L.nnz / G);
+        const bool reuse = A->L.n_rows > kRangeMinRows * G && 2 * shared < units && (int64_t)SL->max_win[mixed_arith] <= 4 * (A->L.nnz / G);
         if (kw && (G == 1 || reuse) && need + 4096 <= (size_t)A->max_lds) {
             k = kw;
             lds = need;
