@@ -557,7 +557,8 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
     // every launch starts from x = 0 (the reset clears x with the publish buffers), and
     // the batched core has neither the transposed streams nor the dynamic classes
     if (o.use_x0 || o.transpose || o.dynamic_precision) return MF_ERR_UNSUPPORTED;
-    bool mixed = o.precision == MF_PREC_MIXED && A->L.has_lowp;
+    const bool asked = o.precision == MF_PREC_MIXED && A->L.has_lowp;
+    bool mixed = asked;
     const int rpt = B->rows_per_wg / 1024;
     BatchKernel k = mixed ? pick_batch<true>(rpt, B->unroll) : pick_batch<false>(rpt, B->unroll);
     if (!k) return MF_ERR_INVALID;
@@ -593,7 +594,6 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
             };
             const SellLayout &SL = *layout;
             const bool narrow = SL.narrow;
-            const bool asked = mixed;
             int64_t low = 0;
             for (int c = 0; c < mfk::kSellAll64; c++) low += SL.units[c];
             if (o.layout == 0 && (double)SL.units[mfk::kSellAll64] <= kBatchUnits64 * (double)low) mixed = false;
@@ -727,7 +727,13 @@ extern "C" mf_status mf_cg_solve_batched(mf_batch *B, const double *d_b, double 
         return MF_ERR_HIP;
     int worst = MF_SUCCESS;
     for (int sidx = 0; sidx < B->count; sidx++) {
-        const double *f = h.data() + (size_t)8 * sidx;
+        double *f = h.data() + (size_t)8 * sidx;
+        // (as in the single-system launcher: r = 0 in binary64 within a fixed number of
+        // iterations of a tile-mixed request)
+        if (o.fixed_iterations && asked && !mixed && (int)f[4] == MF_BREAKDOWN && f[1] == 0.0) {
+            f[0] = o.max_iter;
+            f[4] = MF_SUCCESS;
+        }
         const int status = (int)f[4];
         if (status != MF_SUCCESS && worst == MF_SUCCESS) worst = status;
         if (status == MF_TIMEOUT) worst = MF_TIMEOUT;

@@ -258,8 +258,8 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     if (A->L.tilem == 0) return MF_ERR_INVALID;
     // (pipelined CG holds five row vectors: at most 2 rows per thread, so the chunk rule)
     const long long tuned = ((long long)(req ? req : 2) << 8) | (mixed ? 1 : 0);
-    const bool tiny = tiny_ok && (!ext || one_group_plan(A)) && o->grid == 0 && A->tuned_grid.find(tuned) == A->tuned_grid.end() &&
-                      (o->variant == 0 || o->variant == 4) && !dyn && o->layout != 1 && o->value_cache == 0 &&
+    const bool tiny = tiny_ok && (!ext || one_group_plan(A)) && o->grid == 0 &&
+                      A->tuned_grid.find(tuned) == A->tuned_grid.end() && (o->variant == 0 || o->variant == 4) && !dyn && o->layout != 1 && o->value_cache == 0 &&
                       A->L.n_rows <= kTinyRows && A->L.nnz <= kTinyNnz;
     const int G = tiny ? 1 : choose_grid(A, o, tuned, dyn || req == 3 ? 0 : 1024);
     if (G > A->L.tilem) return MF_ERR_INVALID;
@@ -437,6 +437,12 @@ mf_status cg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_solve
     double h[32];
     if ((st = launch_persistent_ws(A, w, k, a, G, B, lds, s, ext ? nullptr : &ms, h)) != MF_SUCCESS) return st;
     const double bb = h[2];
+    // A tile-mixed request that ran binary64 arithmetic may reach r = 0, where its rounded
+    // products did not: of a fixed number of iterations the rest leaves x as it is.
+    if (o->fixed_iterations && mixed && !mixed_arith && (int)h[4] == MF_BREAKDOWN && h[1] == 0.0) {
+        h[0] = o->max_iter;
+        h[4] = MF_SUCCESS;
+    }
     if (info) {
         memset(info, 0, sizeof(*info));
         info->iterations = (int)h[0];
