@@ -211,7 +211,9 @@ typedef struct mf_solve_options {
                               batched CG 1e-5 under lossless classes, else 1e-3; 1e-3 for
                               BiCGSTAB and the multi-kernel solvers) */
     int max_replacements;  /* 0 = default 64 */
-    int grid;              /* 0 = autotuned; else workgroups (must be co-resident) */
+    int grid;              /* 0 = autotuned, or the default (single-kernel CG: systems of at most
+                              2,048 rows and 16,384 entries on one workgroup, others on 64 to
+                              one per CU); else workgroups (must be co-resident) */
     int block;             /* 0 = default (1024) */
     int variant;           /* 0 = default (4; 2 under dynamic classes);
                               1 = textbook (3 grid syncs/iteration);
@@ -227,19 +229,24 @@ typedef struct mf_solve_options {
     double watchdog_ms;    /* grid-barrier wait bound (0 = default 10000 ms) */
     int transpose;         /* solve A^T x = b: the solver runs on A^T as a tiled matrix of its
                               own (same class policy), built on the matrix's first transposed
-                              call from the host copy of its CSR and kept until
-                              mf_matrix_update_values (the reference's CSR transpose,
-                              utils.h:172) */
-    int layout;            /* single-kernel CG / BiCGSTAB SpMV layout: 0 = default (row-per-lane
-                              sliced-ELL streams for tile-mixed CG, for BiCGSTAB, and for
-                              all-FP64 CG whose binary64 stream fits in LDS; tile chunks for
-                              the other all-FP64 CG);
-                              1 = tile chunks; 2 = sliced-ELL.  Sliced-ELL needs static classes
-                              and every column within 32767 - 1024 (rows per thread - 1) of
-                              its row; otherwise the tile chunks are used. */
-    int value_cache;       /* 0 = default: a variant-4 sliced-ELL CG whose workgroups' value
-                              streams fit their LDS next to x copies them there at launch
-                              (info->layout + 4); 1 = always read them from memory */
+                              call from the host copy of its CSR and kept until the
+                              values change (mf_matrix_update_values or its device form; the
+                              reference's CSR transpose, utils.h:172) */
+    int layout;            /* SpMV layout: 0 = default (row-per-lane sliced-ELL streams for
+                              tile-mixed CG, for BiCGSTAB, for all-FP64 CG whose binary64
+                              stream fits in LDS or whose tiles hold few entries, and for the
+                              multi-kernel solvers where rows pad little; tile chunks for the
+                              other all-FP64 CG; a tile-mixed CG or batch runs binary64
+                              arithmetic where that is the faster, see info->precision);
+                              1 = tile chunks; 2 = sliced-ELL at the tile classes.  Sliced-ELL
+                              needs static classes and every column within
+                              32767 - 1024 (rows per thread) of its row; otherwise the tile
+                              chunks are used. */
+    int value_cache;       /* 0 = default: a variant-4 sliced-ELL CG, or an all-FP64 BiCGSTAB,
+                              whose workgroups' value streams fit their LDS next to the vectors
+                              copies them there at launch (info->layout + 4), and small systems
+                              may run on one workgroup; 1 = always read the values from memory,
+                              on the grid of larger systems */
 } mf_solve_options;
 
 typedef struct mf_solve_info {

@@ -481,7 +481,10 @@ using BatchKernel = void (*)(mfk::BatchArgs);
 // batch runs binary64 arithmetic.  Its SpMV waits for units, not bytes, and class streams
 // start their pipelines one after another: shifted Laplacians (3 units of two class streams
 // for 3 or 4) take 9.9 us an iteration in binary64 and 11.7 tile-mixed in groups of sixteen,
-// 4.5 and 5.5 in groups of one, and need no residual replacements.
+// 4.5 and 5.5 in groups of one, and need no residual replacements.  The rule holds where the
+// streams leave the caches (200 x 40^3, 1 GB of binary64: 19.5 against 20.9 ms; 64 x 256^2 5.3
+// against 6.2) and for one binary32 class stream of 2 units for 3 (512 x 33^2 0.76 against
+// 0.91 ms, 24 x 360^2 4.46 against 4.47).
 constexpr double kBatchUnits64 = 1.5;
 
 // Most window columns per row with which a member gathers p from an LDS window: stencil

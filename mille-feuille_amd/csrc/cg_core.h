@@ -155,7 +155,8 @@ __device__ __forceinline__ void publish_p(const CgPart &a, Rows<RPT, BLK> &R, co
 
 // The window's columns outside this workgroup's own rows: read from the published p
 // (agent-scope loads; every owner's publish is known to be complete), eight in flight a
-// thread, or zero when no other workgroup exists (no column outside the rows then).
+// thread; columns outside the vector's bounds read 0.  Not called when no other workgroup
+// exists.
 template <int BLK, bool W32>
 __device__ __forceinline__ void win_halo(const CgPart &a, int row0, int nrows)
 {
@@ -489,8 +490,8 @@ __device__ CgResult cg_core(const CgPart &a, Rows<RPT, BLK> &R, Sync &sy, double
 // while another workgroup still gathers it.  The tests of an iteration run after its
 // SpMV (whose product is then discarded on exit or replacement), so iteration counts are
 // those of the textbook recurrence.  A replacement (tile-mixed) publishes the corrected
-// p with a grid barrier and redoes the iteration.  Only the single-system kernel (all
-// workgroups of the launch) uses it.
+// p with a grid barrier and redoes the iteration.  The single-system kernel runs it on all
+// workgroups of the launch, the batched kernel on a system's group.
 // Thread slots past the range carry r = p = q = 0 through the dot products and the update
 // instead of being branched around: with a branch per row the compiler kept p in one block
 // of registers and copied all of it, 16 moves each way, around every row's update (at 8

@@ -4,8 +4,8 @@
 // The tile-chunk SpMV adds every entry into LDS (ds_add_f64) and stays near 3 TB/s whatever
 // its block size, depth and grid (3D 127 x 129 x 125 binary64: 52 to 57 us); here a lane sums
 // its own row in a register and a wave's slot is independent of every other, so the kernel
-// only waits for its stream (35.8 us, 4.7 TB/s of the stream and the vectors; tile-mixed 63 ->
-// 28 us).  Used where rows pad little (rows_padding); matrices with rows of
+// only waits for its stream (35.8 us, 4.3 TB/s of the values, a byte of index and the vectors;
+// tile-mixed 63 -> 28 us).  Used where rows pad little (rows_padding); matrices with rows of
 // very different lengths keep the tile chunks.
 #include <hip/hip_runtime.h>
 

@@ -478,7 +478,8 @@ mf_status bicg_launch(mf_matrix *A, const double *d_b, double *d_x, const mf_sol
         k = mixed_arith ? (narrow ? pick_bicg<1, 2>(rpt) : pick_bicg<1, 1>(rpt)) : pick_bicg<0, 1>(rpt);
     // An all-FP64 solve whose binary64 stream fits the workgroups' LDS next to x and v holds it
     // there: both products of an iteration (and the residual checks) then wait for their
-    // gathers only (3D convection-diffusion 63 x 65 x 61: 2.17 -> 2.05 ms).
+    // gathers only (3D convection-diffusion, value_cache off / on in turn: 40 x 41 x 42
+    // 1.089 / 1.082 ms, 63 x 65 x 61 2.118 / 1.994, 70^3 2.453 / 2.184, 78^3 3.93 / 2.79).
     bool on_chip = false;
     if (k && sell && !mixed_arith && !dsell.perm && o->value_cache == 0) {
         size_t offs[mfk::kSellStreams];

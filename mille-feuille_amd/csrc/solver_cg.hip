@@ -225,8 +225,8 @@ int default_grid(const mf_matrix *A, int maxG, int cg_rows)
     }
     // small systems: fewer workgroups make the grid syncs cheaper, but not fewer than 64
     // (8 per XCD): below that the SpMV of each workgroup costs more than the exchanges it
-    // saves (FP64 CG on 2D Poisson 64 x 64: 1.48 ms on 64 workgroups, 1.96 ms on 7;
-    // 128 x 128: 3.12 ms on 64, 3.86 ms on 27)
+    // saves (FP64 CG on 2D Poisson 64 x 64: 0.87 ms on 64 workgroups, 0.83 on 16, 0.93 on 7;
+    // 90 x 91: 1.37 on 64, 1.40 on 16; 128 x 128: 1.73 on 64, 1.96 on 27)
     long long per = 256;  // chunks per workgroup below which the grid shrinks
     long long g = (A->L.nchunks + per - 1) / per;
     g = std::max<long long>(g, 64);
